@@ -152,6 +152,63 @@ def test_rollback_restores_history_and_rng(ctx):  # sampler.rs:348-372 on the de
     assert s.sample(logits) == clean.sample(logits)
 
 
+@pytest.mark.parametrize("kind,n,kw", [
+    # the kept values by list: parts of 1024 values, their remainders, one value past
+    ("normal", 1023, dict(top_k=1, top_p=0.7)),
+    ("normal", 1025, dict(top_k=1024)),
+    ("normal", 4097, dict(top_k=600, top_p=0.999)),   # more than 512 kept: the one-wave sums
+    ("normal", 2048, dict(top_k=30, top_p=0.0)),
+    ("normal", 2048, dict(top_k=30, top_p=NAN)),
+    ("normal", 70001, dict(top_k=3000, top_p=0.9)),
+    ("wide", 5000, dict(top_k=64, top_p=0.95)),       # exps that underflow among the kept
+    # ties at the threshold: within the list, and more than it holds
+    ("ties", 3000, dict(top_k=40, top_p=0.5)),
+    ("ties", 9000, dict(top_k=40, top_p=0.5)),
+    ("zeros", 3000, dict(top_k=10)),                  # +0 and -0 around the threshold
+    ("zeros", 9000, dict(top_k=10, top_p=0.4)),
+    ("neg_inf", 3000, dict(top_k=100, top_p=0.9)),    # fewer finite values than k
+    # all values: chunks of 512 terms, rounds of 262144
+    ("normal", 511, dict(top_p=0.9)),
+    ("normal", 513, dict()),
+    ("wide", 20000, dict(top_p=0.99)),
+    ("sparse", 60000, dict()),                        # chunks of zeros, before the first term too
+    ("normal", 262145, dict(top_p=0.8)),
+    ("normal", 300001, dict(repetition_penalty=1.2)),
+])
+def test_sample_routes_match_oracle(ctx, kind, n, kw):
+    """Top-k through the list or the sort, and the sums over all values by
+    chunks: the oracle's ids at the sizes where the routes and their parts
+    change, with a history that reaches the device in a copy (40 ids) and then
+    id by id, duplicates among them."""
+    print(f"sampler route {kind} n={n} {kw}", flush=True)
+    rng = np.random.default_rng(n)
+    kw = dict(temperature=0.9, **{"repetition_penalty": 1.15, **kw})
+    dev, ref = pair_samplers(ctx, 4321 + n, **kw)
+    for tok in rng.integers(0, n, 40).tolist() + [0, n - 1, n + 5]:
+        dev.observe(tok)
+        ref.observe(tok)
+    for step in range(4):
+        x = (rng.standard_normal(n) * 2).astype(np.float32)
+        if kind == "wide":
+            x *= np.float32(40)
+        elif kind == "ties":
+            x = np.round(x * np.float32(0.25))
+        elif kind == "zeros":
+            x = np.where(rng.random(n) < 0.5, 0.0, -0.0).astype(np.float32)
+            x[::500] = 1.0
+        elif kind == "neg_inf":
+            x[rng.permutation(n)[50:]] = -np.inf
+        elif kind == "sparse":
+            x[:40000] = -300.0
+            x[rng.permutation(n)[1000:]] = -300.0
+            x[50000] = 3.0
+        got, want = dev.sample(x), ref.sample(x)
+        assert got == want, f"step {step}"
+        assert dev.checkpoint()[0] == ref.state.value
+        dev.observe(got)
+        ref.observe(want)
+
+
 # ---- batched prefill and the sampled loop --------------------------------
 
 LONG = bs.BitNetConfig(n_layers=2, n_embd=256, n_ff=384, n_heads=4, n_kv_heads=2, head_dim=64,
