@@ -648,85 +648,124 @@ struct attn_rows_args {
     const wm_attn_item *sc_items, *sv_items;  // work items of the scores and V kernels
 };
 
-constexpr int kScoreThreads = 256;  // positions per scores item, one per thread
-constexpr int kScoreTok = 8;        // tokens (of one sequence) per scores item
+constexpr int kScoreThreads = 256;      // positions per scores item, one per thread
+constexpr uint32_t kScoreTokMax = 8;    // tokens (of one sequence) per scores item, at most
 
-// scores[t][h][p] for the NT tokens t0 .. t0+NT-1 of one sequence (item
-// it), the G query heads of the item's KV head and position p (this thread):
-// the thread loads its K row once, dequantises it (read_into: q8 * scale) and
-// runs the NT*G chains Σ_i q[i] * k[i], each in dimension order, then
-// * (1/sqrt(head_dim)).  The query values are the same for every lane and
-// are read as scalars.  Positions past a token's own are computed from rows
-// other tokens of the batch have written and never read.
 // Memory that no thread writes while the kernel runs, addressed so that the
 // compiler may read it through the scalar unit wherever the address is the
 // same for every lane.
 typedef const float __attribute__((address_space(4))) wm_const_f32;
 
-template <int HD, int G, int NT>
-__device__ __forceinline__ void scores_item(const int8_t *kp, float kscale, const float *qb,
-                                            uint64_t qstride, float *dst, uint64_t sstride,
-                                            float scale) {
-    float s[NT][G];
-#pragma unroll
-    for (int tt = 0; tt < NT; tt++)
-#pragma unroll
-        for (int g = 0; g < G; g++) s[tt][g] = 0.0f;
-    // the next 16 codes are in flight while the current ones are used
-    int4 raw = *reinterpret_cast<const int4 *>(kp);
-#pragma unroll 1
-    for (int b = 0; b < HD / 16; b++) {
-        const int4 cur = raw;
-        if (b + 1 < HD / 16) raw = *reinterpret_cast<const int4 *>(kp + (b + 1) * 16);
-        float kd[16];
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-            const uint32_t wd = e < 4 ? (uint32_t)cur.x : e < 8 ? (uint32_t)cur.y : e < 12 ? (uint32_t)cur.z : (uint32_t)cur.w;
-            kd[e] = (float)(int8_t)(wd >> (8 * (e & 3))) * kscale;  // read_into
-        }
-#pragma unroll
-        for (int tt = 0; tt < NT; tt++) {
-            const wm_const_f32 *qt = (const wm_const_f32 *)qb + (uint64_t)tt * qstride + b * 16;
-#pragma unroll
-            for (int g = 0; g < G; g++)
-#pragma unroll
-                for (int e = 0; e < 16; e++) s[tt][g] = s[tt][g] + qt[g * HD + e] * kd[e];
-        }
-    }
-    // token tt, head g: dst[(tt * G + g) * sstride] (the token's rows follow
-    // its G heads' rows: n_heads rows per token, G of them this KV head's)
-#pragma unroll
-    for (int tt = 0; tt < NT; tt++)
-#pragma unroll
-        for (int g = 0; g < G; g++) dst[(uint64_t)tt * qstride / HD * sstride + (uint64_t)g * sstride] = s[tt][g] * scale;
-}
-
-// One item per workgroup (blockIdx.x): its nt (1 .. kScoreTok) tokens and
-// positions p0 .. p0+255 below p1, one position per thread.
+// scores[t][h][p] for the nt tokens t0 .. t0+nt-1 of one sequence (item
+// blockIdx.x), the G query heads of KV head `unit` and the positions p0 ..
+// p0+255 below p1, one per thread: the thread dequantises its K row once
+// (read_into: q8 * scale) and runs the nt*G chains Σ_i q[i] * k[i], each in
+// dimension order, then * (1/sqrt(head_dim)).  Positions past a token's own
+// are computed from rows other tokens of the batch have written and never
+// read.
+// Bound by VALU issue: each term is a separately rounded multiply and add,
+// and the query values, the same for every lane, are scalar operands.  Eight
+// dimensions of four rows (32 scalars) are used while the next eight are in
+// flight, across the rows' ends too; read where they were used, the waits
+// for them took half the time.  (As DPP broadcasts from vector registers the
+// multiplies issue at 0.4 of the plain rate.)  Per BitNet-2B layer: 512
+// prompt tokens from an empty cache 80 -> 32 us, 32 tokens at context 3000 69
+// -> 22 (both with the placement below), 16 ragged sequences (293 tokens,
+// contexts to 4000) 106 -> 94; the multiplies and adds alone take 11, 9 and
+// 46 us at the rate a loop of them reaches.
 template <int HD, int G>
-__global__ __launch_bounds__(kScoreThreads) void k_attn_scores_rows(attn_rows_args a) {
-    static_assert(kScoreTok == 8, "one case per token count");
+__global__ __launch_bounds__(kScoreThreads, 2) void k_attn_scores_rows(attn_rows_args a) {
     const wm_attn_item it = a.sc_items[blockIdx.x];
     const uint32_t p = it.p0 + threadIdx.x;
-    if (it.nt == 0 || p >= it.p1) return;
-    const uint32_t kvh = it.unit;
+    if (it.nt == 0 || (p & ~63u) >= it.p1) return;  // (p0 is a multiple of 64: whole waves)
+    const uint32_t kvh = it.unit, rows = it.nt * G;
     const wm_batch_tok tk = a.tok[it.t0];  // every token of the item: the same cache
     const uint64_t lay = (uint64_t)a.layer * tk.max_seq;
-    const int8_t *kp = tk.k + (lay + p) * a.kv_dim + kvh * HD;
-    const float kscale = tk.ks[lay + p];
-    const float *qb = a.q + (uint64_t)it.t0 * a.n_heads * HD + (uint64_t)kvh * G * HD;
-    const uint64_t qstride = (uint64_t)a.n_heads * HD;
+    // row r: head r % G of token r / G; four rows at a time (a row past the
+    // last: the last again, not stored)
+    const wm_const_f32 *q0 = (const wm_const_f32 *)a.q + ((uint64_t)it.t0 * a.n_heads + kvh * G) * HD;
+    const auto row_off = [&](uint32_t r) { return (uint64_t)(r / G) * a.n_heads + r % G; };
+    const uint32_t r_last = (rows - 1) & ~3u;
+    struct q_block {
+        float v[4][8];
+    };
+    const auto q_load = [&](q_block &q, uint32_t r0, int d) {
+        const wm_const_f32 *qr[4];
+        if constexpr (G % 4 == 0) {  // heads of one token: consecutive rows
+            qr[0] = q0 + row_off(r0) * HD + d;
+            // (opaque, so that two blocks' loads are not merged: the scalar
+            // registers hold two blocks, not four)
+            asm volatile("" : "+s"(qr[0]));
+#pragma unroll
+            for (uint32_t i = 1; i < 4; i++) qr[i] = qr[0] + i * HD;
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) {
+                qr[i] = q0 + row_off(min(r0 + i, rows - 1)) * HD + d;
+                asm volatile("" : "+s"(qr[i]));
+            }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) q.v[i][e] = qr[i][e];
+    };
+    q_block qa, qb;
+    q_load(qa, 0, 0);
+    float kd[HD];
+    {
+        const uint32_t pc = min(p, it.p1 - 1);  // (a thread past the end computes the last position, not stored)
+        const int8_t *kp = tk.k + (lay + pc) * a.kv_dim + kvh * HD;
+        const float kscale = tk.ks[lay + pc];
+        int4 raw[HD / 16];
+#pragma unroll
+        for (int b = 0; b < HD / 16; b++) raw[b] = *reinterpret_cast<const int4 *>(kp + b * 16);
+#pragma unroll
+        for (int i = 0; i < HD; i++) {
+            const int4 c = raw[i / 16];
+            const int e = i % 16;
+            const uint32_t wd = e < 4 ? (uint32_t)c.x : e < 8 ? (uint32_t)c.y : e < 12 ? (uint32_t)c.z : (uint32_t)c.w;
+            kd[i] = (float)(int8_t)(wd >> (8 * (e & 3))) * kscale;  // read_into
+        }
+    }
     float *dst = a.scores + ((uint64_t)it.t0 * a.n_heads + kvh * G) * a.score_stride + p;
-    const uint64_t ss = a.score_stride;
-    switch (it.nt) {
-        case 1: scores_item<HD, G, 1>(kp, kscale, qb, qstride, dst, ss, a.scale); break;
-        case 2: scores_item<HD, G, 2>(kp, kscale, qb, qstride, dst, ss, a.scale); break;
-        case 3: scores_item<HD, G, 3>(kp, kscale, qb, qstride, dst, ss, a.scale); break;
-        case 4: scores_item<HD, G, 4>(kp, kscale, qb, qstride, dst, ss, a.scale); break;
-        case 5: scores_item<HD, G, 5>(kp, kscale, qb, qstride, dst, ss, a.scale); break;
-        case 6: scores_item<HD, G, 6>(kp, kscale, qb, qstride, dst, ss, a.scale); break;
-        case 7: scores_item<HD, G, 7>(kp, kscale, qb, qstride, dst, ss, a.scale); break;
-        default: scores_item<HD, G, 8>(kp, kscale, qb, qstride, dst, ss, a.scale); break;
+#pragma unroll 1
+    for (uint32_t r0 = 0; r0 < rows; r0 += 4) {
+        float s[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) s[i] = 0.0f;
+        const auto add8 = [&](const q_block &q, int d) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) s[i] = s[i] + q.v[i][e] * kd[d + e];
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // Scalar loads return in any order, so a wait for one is a wait for
+        // all: the block about to be used is waited for (it had the block
+        // before it to arrive) before the next one's loads go out.
+        const auto wait_q = [&]() {
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0) alone
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int d = 0; d < HD; d += 16) {
+            wait_q();
+            q_load(qb, r0, d + 8);
+            __builtin_amdgcn_sched_barrier(0);  // the loads go out before these terms
+            add8(qa, d);
+            wait_q();
+            if (d + 16 < HD) q_load(qa, r0, d + 16);
+            else q_load(qa, min(r0 + 4, r_last), 0);  // the next rows'
+            __builtin_amdgcn_sched_barrier(0);
+            add8(qb, d + 8);
+        }
+        // (the chains end here, not inside the branch)
+        asm volatile("" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
+        if (p < it.p1)
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++)
+                if (r0 + i < rows) dst[row_off(r0 + i) * a.score_stride] = s[i] * a.scale;
     }
 }
 
@@ -1024,6 +1063,7 @@ __global__ __launch_bounds__(HD) void k_attn_sv_rows(attn_rows_args a) {
 
 namespace {
 constexpr uint32_t kGemmCus = 256;
+constexpr uint32_t kAttnSimds = 4 * kGemmCus;
 }  // namespace
 
 wm_gemm_plan wm_gemm_make_plan(uint32_t groups, uint32_t n_chunks, uint32_t m) {
@@ -1145,65 +1185,97 @@ wm_attn_item *wm_attn_rows_items(float *scores, uint32_t m, uint32_t n_heads, ui
 
 uint32_t wm_attn_rows_sv_parts(uint32_t group) { return group < kSvHeads ? 1u : group / kSvHeads; }
 
-// Items in launch order.  Workgroup i runs on XCD i % 8, so the items of one
-// (sequence, unit) group, which read the same K or V rows, are all given
-// the same i % 8 and share that XCD's L2; groups go to the least-loaded XCD,
-// largest first, and the shorter lists are padded with empty items.
-static void attn_place(std::vector<std::vector<wm_attn_item>> &groups, std::vector<uint64_t> &work,
-                       std::vector<wm_attn_item> &out) {
-    constexpr uint32_t kXcds = 8;
-    std::vector<uint32_t> order(groups.size());
-    for (uint32_t i = 0; i < order.size(); i++) order[i] = i;
-    std::sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return work[x] > work[y]; });
-    std::vector<std::vector<wm_attn_item>> lists(kXcds);
+// Workgroup i runs on XCD i % 8.  The items of one (sequence, unit) read the
+// same K or V rows, so they share an XCD's L2 while that leaves the XCDs
+// evenly loaded: a group of items is cut into pieces of at most 1/32 of the
+// work, and each piece goes to the least-loaded XCD, largest first (a single
+// sequence has one group per KV head: uncut, its five groups left three XCDs
+// idle).  An XCD's items run in order of their work, the longest first; the
+// shorter lists are padded with empty items.
+struct attn_piece {
+    uint64_t work;
+    uint32_t first, n;  // items [first, first + n)
+};
+static void attn_place(const std::vector<wm_attn_item> &items, const std::vector<uint64_t> &work,
+                       const std::vector<uint32_t> &group, std::vector<wm_attn_item> &out) {
+    constexpr uint32_t kXcds = 8, kPieces = 32;
+    uint64_t total = 0;
+    for (uint64_t w : work) total += w;
+    std::vector<attn_piece> pieces;
+    for (uint32_t i = 0; i < items.size(); i++) {
+        if (i == 0 || group[i] != group[i - 1] || (pieces.back().work + work[i]) * kPieces > total)
+            pieces.push_back({0, i, 0});
+        pieces.back().work += work[i];
+        pieces.back().n++;
+    }
+    std::stable_sort(pieces.begin(), pieces.end(),
+                     [](const attn_piece &x, const attn_piece &y) { return x.work > y.work; });
+    std::vector<uint32_t> lists[kXcds];
     uint64_t load[kXcds] = {};
-    for (uint32_t g : order) {
+    for (const attn_piece &p : pieces) {
         uint32_t x = 0;
         for (uint32_t k = 1; k < kXcds; k++)
             if (load[k] < load[x]) x = k;
-        load[x] += work[g];
-        lists[x].insert(lists[x].end(), groups[g].begin(), groups[g].end());
+        load[x] += p.work;
+        for (uint32_t i = 0; i < p.n; i++) lists[x].push_back(p.first + i);
     }
     size_t len = 0;
-    for (auto &l : lists) len = std::max(len, l.size());
+    for (auto &l : lists) {
+        std::stable_sort(l.begin(), l.end(), [&](uint32_t x, uint32_t y) { return work[x] > work[y]; });
+        len = std::max(len, l.size());
+    }
     out.assign(len * kXcds, wm_attn_item{0, 0, 0, 0, 0, 0});
     for (uint32_t x = 0; x < kXcds; x++)
-        for (size_t k = 0; k < lists[x].size(); k++) out[k * kXcds + x] = lists[x][k];
+        for (size_t k = 0; k < lists[x].size(); k++) out[k * kXcds + x] = items[lists[x][k]];
 }
 
 void wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t sc_units, uint32_t sv_units,
                        std::vector<wm_attn_item> &sc, std::vector<wm_attn_item> &sv) {
-    std::vector<std::vector<wm_attn_item>> sc_groups, sv_groups;
-    std::vector<uint64_t> sc_work, sv_work;
+    // the sequences: tokens of one cache at consecutive positions
+    std::vector<std::pair<uint32_t, uint32_t>> seqs;
     for (uint32_t t = 0; t < m;) {
-        uint32_t e = t + 1;  // the sequence's tokens: same cache, consecutive positions
+        uint32_t e = t + 1;
         while (e < m && tok[e].k == tok[t].k && tok[e].pos == tok[e - 1].pos + 1) e++;
-        for (uint32_t u = 0; u < sc_units; u++) {
-            std::vector<wm_attn_item> g;
-            uint64_t w = 0;
-            for (uint32_t b = t; b < e; b += kScoreTok) {
-                const uint32_t nt = std::min<uint32_t>(kScoreTok, e - b), p1 = tok[b + nt - 1].pos + 1;
-                for (uint32_t p0 = 0; p0 < p1; p0 += kScoreThreads) g.push_back({b, nt, p0, p1, u, 0});
-                w += (uint64_t)nt * p1;
-            }
-            sc_groups.push_back(g);
-            sc_work.push_back(w);
-        }
-        for (uint32_t u = 0; u < sv_units; u++) {
-            std::vector<wm_attn_item> g;
-            uint64_t w = 0;
-            for (uint32_t b = t; b < e; b += kSvTok) {
-                const uint32_t nt = std::min<uint32_t>(kSvTok, e - b), p1 = tok[b + nt - 1].pos + 1;
-                g.push_back({b, nt, 0, p1, u, 0});
-                w += (uint64_t)nt * p1;
-            }
-            sv_groups.push_back(g);
-            sv_work.push_back(w);
-        }
+        seqs.emplace_back(t, e);
         t = e;
     }
-    attn_place(sc_groups, sc_work, sc);
-    attn_place(sv_groups, sv_work, sv);
+    // Tokens per scores item: as many as leave three waves per SIMD (a K row
+    // is dequantised once per item, its share small from four tokens on).
+    uint32_t nt_max = kScoreTokMax;
+    for (; nt_max > 1; nt_max /= 2) {
+        uint64_t waves = 0;
+        for (auto &q : seqs)
+            for (uint32_t b = q.first; b < q.second; b += nt_max)
+                waves += (uint64_t)sc_units * (tok[std::min(b + nt_max, q.second) - 1].pos / 64 + 1);
+        if (waves >= 3 * kAttnSimds) break;
+    }
+    std::vector<wm_attn_item> items;
+    std::vector<uint64_t> work;
+    std::vector<uint32_t> group;
+    uint32_t gid = 0;
+    for (auto &q : seqs)
+        for (uint32_t u = 0; u < sc_units; u++, gid++)
+            for (uint32_t b = q.first; b < q.second; b += nt_max) {
+                const uint32_t nt = std::min(nt_max, q.second - b), p1 = tok[b + nt - 1].pos + 1;
+                for (uint32_t p0 = 0; p0 < p1; p0 += kScoreThreads) {
+                    items.push_back({b, nt, p0, p1, u, 0});
+                    work.push_back((uint64_t)nt * std::min<uint32_t>(kScoreThreads, p1 - p0));
+                    group.push_back(gid);
+                }
+            }
+    attn_place(items, work, group, sc);
+    items.clear();
+    work.clear();
+    group.clear();
+    for (auto &q : seqs)
+        for (uint32_t u = 0; u < sv_units; u++, gid++)
+            for (uint32_t b = q.first; b < q.second; b += kSvTok) {
+                const uint32_t nt = std::min<uint32_t>(kSvTok, q.second - b), p1 = tok[b + nt - 1].pos + 1;
+                items.push_back({b, nt, 0, p1, u, 0});
+                work.push_back((uint64_t)nt * p1);
+                group.push_back(gid);
+            }
+    attn_place(items, work, group, sv);
 }
 
 void wm_launch_attn_rows(const float *q, const wm_batch_tok *tok, uint32_t m, uint32_t n_max,

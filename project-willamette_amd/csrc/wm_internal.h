@@ -569,9 +569,9 @@ struct wm_attn_item {
     uint32_t t0, nt, p0, p1, unit, pad;
 };
 // From the step's tokens (host copy; a sequence's tokens are consecutive):
-// scores items per (sequence, KV head, 8 tokens, 256 positions) and V items
-// per (sequence, KV-head part, token), ordered so that every item of one
-// (sequence, unit) runs on the same XCD.
+// scores items per (sequence, KV head, up to 8 tokens, 256 positions) and V items
+// per (sequence, KV-head part, token), ordered so that the XCDs share the
+// work evenly and items that read the same rows share an XCD where they can.
 void wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t sc_units, uint32_t sv_units,
                        std::vector<wm_attn_item> &sc, std::vector<wm_attn_item> &sv);
 // V-kernel units per KV head for a query group size
