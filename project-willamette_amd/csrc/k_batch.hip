@@ -627,23 +627,22 @@ __global__ __launch_bounds__(256) void k_qkv_rows(qkv_rows_args a) {
 
 // ---------------------------------------------------------------------------
 // causal GQA attention of every token over its own sequence
-// (cached_forward.rs:417-449, attention.rs:45-73), in two kernels
+// (cached_forward.rs:417-449, attention.rs:45-73), in three kernels
 // ---------------------------------------------------------------------------
 //
 // Scores: one thread per (position, KV head) computes the G query heads'
 // 128-term dots from one K row, each in order with k = q8 * scale, then
 // * (1/sqrt(head_dim)), into scores[t][h][p].
-// Softmax + V: one workgroup per (token, head): max, exp (glibc expf), exact
-// sequential sum, * (1/sum), then one thread per output dimension runs
-// Σ_p w_p * v_p[d] in position order.
+// Softmax: per (token, head) max, exp (glibc expf), exact sequential sum,
+// * (1/sum).
+// V: one lane per output dimension runs Σ_p w_p * v_p[d] in position order.
 struct attn_rows_args {
     const float *q;  // [t][n_heads * head_dim]
     const wm_batch_tok *tok;
-    float *scores;   // [t][n_heads][score_stride]: the scores, then exp(s - max)
+    float *scores;   // [t][n_heads][score_stride]: the scores, then the weights
     float *out;      // [t][n_heads * head_dim]
     uint32_t layer, kv_dim, n_heads, score_stride, n_max;
     float scale;
-    float *row_scale;  // [t][n_heads]: 1 / Σexp (1 when Σ is not positive)
     uint8_t *live;     // [t][n_heads][kAttnTiles]: the tile of kSvPos positions holds a non-zero exp
     const wm_attn_item *sc_items, *sv_items;  // work items of the scores and V kernels
 };
@@ -655,6 +654,11 @@ constexpr uint32_t kScoreTokMax = 8;    // tokens (of one sequence) per scores i
 // compiler may read it through the scalar unit wherever the address is the
 // same for every lane.
 typedef const float __attribute__((address_space(4))) wm_const_f32;
+// Global memory, said so: a pointer read from memory is a flat one otherwise,
+// and flat loads count with the scalar loads and LDS operations.
+typedef const int8_t __attribute__((address_space(1))) wm_global_i8;
+typedef const v4i __attribute__((address_space(1))) wm_global_v4i;
+typedef const float __attribute__((address_space(1))) wm_global_f32;
 
 // scores[t][h][p] for the nt tokens t0 .. t0+nt-1 of one sequence (item
 // blockIdx.x), the G query heads of KV head `unit` and the positions p0 ..
@@ -715,14 +719,14 @@ __global__ __launch_bounds__(kScoreThreads, 2) void k_attn_scores_rows(attn_rows
     float kd[HD];
     {
         const uint32_t pc = min(p, it.p1 - 1);  // (a thread past the end computes the last position, not stored)
-        const int8_t *kp = tk.k + (lay + pc) * a.kv_dim + kvh * HD;
-        const float kscale = tk.ks[lay + pc];
-        int4 raw[HD / 16];
+        const wm_global_v4i *kp = (const wm_global_v4i *)(tk.k + (lay + pc) * a.kv_dim + kvh * HD);
+        const float kscale = ((const wm_global_f32 *)tk.ks)[lay + pc];
+        v4i raw[HD / 16];
 #pragma unroll
-        for (int b = 0; b < HD / 16; b++) raw[b] = *reinterpret_cast<const int4 *>(kp + b * 16);
+        for (int b = 0; b < HD / 16; b++) raw[b] = kp[b];
 #pragma unroll
         for (int i = 0; i < HD; i++) {
-            const int4 c = raw[i / 16];
+            const v4i c = raw[i / 16];
             const int e = i % 16;
             const uint32_t wd = e < 4 ? (uint32_t)c.x : e < 8 ? (uint32_t)c.y : e < 12 ? (uint32_t)c.z : (uint32_t)c.w;
             kd[i] = (float)(int8_t)(wd >> (8 * (e & 3))) * kscale;  // read_into
@@ -769,111 +773,73 @@ __global__ __launch_bounds__(kScoreThreads, 2) void k_attn_scores_rows(attn_rows
     }
 }
 
-// out[t][h][d] = Σ_p w_h[p] * v_p[d] in position order (cached_forward.rs:
-// 417-449; v_p[d] = q8 * scale, read_into) for kSvTok tokens of one sequence
-// (item blockIdx.x) and G query heads of one KV head, on the exps
-// k_attn_softmax_rows left in place of the scores times each row's 1/sum.
-// Thread d runs the kSvTok * G chains: they share every V value.  Tiles of
-// kSvPos positions go through LDS: the V codes and scales (the next tile's
-// loads in flight while the current one is summed) and the rows' weights; a
-// token's positions past its own get weight 0 (exact: a zero term leaves
-// the sum unchanged), so every tile runs in full.
-// The pass ends when its longest rows do (heads whose exps are non-zero
-// over the whole context, while most rows have one live tile), and what
-// such a row waits on is its waves' own work per tile; so each workgroup
-// takes one query head, although the heads of a KV group could share the
-// V dequantisation (BitNet-2B, 16 sequences: 133 us per layer with four
-// heads per workgroup, 99 with two, 90 with one).
-constexpr uint32_t kSvPos = 64;
-constexpr uint32_t kSvHeads = 1;  // query heads per workgroup (of one KV head's group)
-constexpr uint32_t kSvTok = 1;    // tokens per V item
-constexpr uint32_t kAttnTiles = 64;  // tiles of kSvPos positions per row (contexts <= 4096)
+constexpr uint32_t kSvPos = WM_ATTN_TILE;  // positions per tile of the V pass
+constexpr uint32_t kAttnTiles = 64;  // tiles per row (contexts <= 4096)
 
-// The loads of V tile rows p0 .. p0 + kSvPos - 1 (indices clamped to n - 1):
-// thread tid takes 16-byte pieces tid, tid + HD, tid + 2HD, tid + 3HD
-// (piece = row * HD/16 + column) and their rows' scales, in named registers
-// (an array would be kept in scratch memory).
-struct sv_regs {
-    int4 v0, v1, v2, v3;
-    float s0, s1, s2, s3;
-};
-template <int HD>
-__device__ __forceinline__ uint32_t sv_row(uint32_t i) { return (i * HD + threadIdx.x) / (HD / 16); }
-template <int HD>
-__device__ __forceinline__ uint32_t sv_col(uint32_t i) { return ((i * HD + threadIdx.x) % (HD / 16)) * 16; }
-template <int HD>
-__device__ __forceinline__ void sv_fetch(sv_regs &r, const int8_t *vg, const float *vsg, uint32_t kv_dim,
-                                         uint32_t p0, uint32_t n) {
-    static_assert(kSvPos * HD / 16 == 4 * HD, "four pieces per thread");
-    const auto piece = [&](uint32_t i) {
-        return *reinterpret_cast<const int4 *>(vg + (uint64_t)min(p0 + sv_row<HD>(i), n - 1) * kv_dim +
-                                               sv_col<HD>(i));
-    };
-    r.v0 = piece(0);
-    r.v1 = piece(1);
-    r.v2 = piece(2);
-    r.v3 = piece(3);
-    r.s0 = vsg[min(p0 + sv_row<HD>(0), n - 1)];
-    r.s1 = vsg[min(p0 + sv_row<HD>(1), n - 1)];
-    r.s2 = vsg[min(p0 + sv_row<HD>(2), n - 1)];
-    r.s3 = vsg[min(p0 + sv_row<HD>(3), n - 1)];
-}
-// the tile's codes into vt[row][col] as loaded, and each row's scale into vst[row]
-template <int HD>
-__device__ __forceinline__ void sv_stage(const sv_regs &r, int8_t (*vt)[HD], float *vst) {
-    *reinterpret_cast<int4 *>(&vt[sv_row<HD>(0)][sv_col<HD>(0)]) = r.v0;
-    *reinterpret_cast<int4 *>(&vt[sv_row<HD>(1)][sv_col<HD>(1)]) = r.v1;
-    *reinterpret_cast<int4 *>(&vt[sv_row<HD>(2)][sv_col<HD>(2)]) = r.v2;
-    *reinterpret_cast<int4 *>(&vt[sv_row<HD>(3)][sv_col<HD>(3)]) = r.v3;
-    if (sv_col<HD>(0) == 0) vst[sv_row<HD>(0)] = r.s0;
-    if (sv_col<HD>(1) == 0) vst[sv_row<HD>(1)] = r.s1;
-    if (sv_col<HD>(2) == 0) vst[sv_row<HD>(2)] = r.s2;
-    if (sv_col<HD>(3) == 0) vst[sv_row<HD>(3)] = r.s3;
-}
-
-// Softmax of one (token, head) row of scores per wave (attention.rs:45-73):
-// max, exp (glibc expf) in place, the exact sequential sum of the exps by the
-// one-wave algorithm (512 exps per step, summed from the registers that
-// computed them) and the row's scale 1/sum (1 when the sum is not positive:
-// the reference leaves the row unnormalised); the V pass forms each weight as
-// exp * scale, the same f32 product the reference's `*= inv` makes.  Tiles of
-// kSvPos positions whose exps are all exactly zero are flagged dead: their
+// Softmax of the scores rows in place (attention.rs:45-73): max, exp (glibc
+// expf), the exact sequential sum of the exps, and each weight exp * (1/sum)
+// (the exp itself when the sum is not positive: the reference leaves the row
+// unnormalised); zeros from the row's end to the end of its tile of kSvPos
+// positions.  Tiles whose exps are all exactly zero are flagged dead: their
 // weights are zero, and a zero term leaves each of the V pass's sums
 // unchanged (those sums start at +0 and can never be -0), so it skips them.
 // A row whose maximum is not finite becomes all zero (its output is then 0).
-// The rows of a workgroup are heads of one token, so its waves have equal
-// work; a row's sum has no barrier and no idle wave, and the many rows of a
-// batch keep every SIMD busy.
-constexpr uint32_t kSmRows = 4;  // rows per workgroup, one per wave
-static_assert(kSvPos % 8 == 0 && wm::kSeqBatch / kSvPos == 8, "a step's tiles are 8-lane groups");
-__global__ __launch_bounds__(kSmRows * 64) void k_attn_softmax_rows(attn_rows_args a) {
+//
+// A row's values stay in the registers of its WPR waves (F4 float4 a lane: n
+// <= 256 WPR F4).  The sum is the plain chain of adds: 1024 positions of every
+// row at a time go through LDS, and wave 0 adds the workgroup's rows side by
+// side, a quarter of its lanes per row, four terms per LDS read, while the
+// next 1024 positions' exps are formed.  The chain costs ~2.4 ns a term and one
+// VALU slot for all the rows; the integer sum per 512-term step it replaces
+// restarts at every binade change and halfway case, several hundred cycles
+// each.  Per BitNet-2B layer (rows x mean context): 10220 x 256 25.8 -> 12.5
+// us, 640 x 3000 25.6 -> 18.4, 5860 x 2000 55 -> 50.
+// (exp of a score minus its row's maximum, so of x <= 0 or a NaN: expf_glibc
+// without its branches.  Below -0x1.9fe368p6 it is +0.)
+__device__ __forceinline__ float exp_nonpos(float x, const uint64_t *tab) {
+    const float y = wm::expf_glibc_core(x < -104.0f ? -104.0f : x, tab);
+    return x < -0x1.9fe368p6f ? 0.0f : y;
+}
+constexpr uint32_t kSmRows = 4;      // rows per workgroup
+constexpr uint32_t kSmChunk = 1024;  // positions of each row in LDS at a time
+template <uint32_t WPR, uint32_t F4>
+__global__ __launch_bounds__(kSmRows * WPR * 64) void k_attn_softmax_rows(attn_rows_args a, uint32_t n_rows) {
+    constexpr uint32_t kSlots = kSmChunk / 256;  // float4 slots of a chunk
+    constexpr uint32_t kMine = kSlots / WPR;     // a wave's slots of a chunk
+    constexpr uint32_t kChunks = (F4 + kMine - 1) / kMine;
+    constexpr uint32_t kBufs = kChunks > 1 ? 2 : 1;
+    static_assert(kSlots % WPR == 0, "a chunk's slots over the row's waves");
+    __shared__ __align__(16) float buf[kBufs][kSmRows][kSmChunk + 4];  // (rows on different banks)
     __shared__ uint64_t exp_tab[32];
+    __shared__ float row_inv[kSmRows], red[kSmRows * WPR];
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    if (tid < 32) exp_tab[tid] = wm::kExp2Tab[tid];
-    __syncthreads();
-    const uint32_t h = blockIdx.x * kSmRows + wid, t = blockIdx.y;
-    if (h >= a.n_heads) return;
-    const uint32_t n = a.tok[t].pos + 1, n_tiles = (n + kSvPos - 1) / kSvPos;  // n_tiles <= 64
-    const uint64_t row = (uint64_t)t * a.n_heads + h;
-    float *w = a.scores + row * a.score_stride;
-    uint8_t *live = a.live + row * kAttnTiles;
-    // The row's float4s below n4 = ceil(n / 4) lie inside it (rows start
-    // 16-byte aligned and score_stride >= n rounded up to 4); indices are
-    // clamped to n4 - 1 and components at n and beyond are masked.
-    const float4 *w4 = reinterpret_cast<const float4 *>(w);
+    const uint32_t r = wid / WPR, part = wid % WPR;  // row of the workgroup, the wave's part of it
+    const uint32_t row0 = blockIdx.x * kSmRows, row = min(row0 + r, n_rows - 1);
+    const bool mine = row0 + r < n_rows;
+    const uint32_t n = a.tok[row / a.n_heads].pos + 1;
+    float *w = a.scores + (uint64_t)row * a.score_stride;
+    // Slot k: positions 256 k + 4 lane .. + 3, of wave k % WPR.  (Rows are
+    // padded to whole tiles, so a float4 that holds a position below n lies
+    // inside the row; indices are clamped to the last such one.)
     const uint32_t n4 = (n + 3) / 4;
+    float4 x[F4];
+#pragma unroll
+    for (uint32_t i = 0; i < F4; i++) {
+        const uint32_t k = i * WPR + part;
+        if (256 * k < n) x[i] = reinterpret_cast<const float4 *>(w)[min(64 * k + lane, n4 - 1)];
+    }
+    uint32_t n_max = 0;  // the workgroup's longest row (rows of one token or of two)
+#pragma unroll
+    for (uint32_t i = 0; i < kSmRows; i++)
+        n_max = max(n_max, a.tok[min(row0 + i, n_rows - 1) / a.n_heads].pos + 1);
+    if (tid < 32) exp_tab[tid] = wm::kExp2Tab[tid];
     float mx = -INFINITY;
-    for (uint32_t q0 = 0; q0 < n4; q0 += 256) {  // lane l: float4s q0 + l + 64i
-        float4 x[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t q = q0 + lane + 64 * i;
-            x[i] = w4[min(q, n4 - 1)];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t p = 4 * (q0 + lane + 64 * i);
+    for (uint32_t i = 0; i < F4; i++) {
+        const uint32_t k = i * WPR + part;
+        if (256 * k < n) {
+            const uint32_t p = 256 * k + 4 * lane;
             mx = wm_max_nonan(mx, p < n ? x[i].x : -INFINITY);
             mx = wm_max_nonan(mx, p + 1 < n ? x[i].y : -INFINITY);
             mx = wm_max_nonan(mx, p + 2 < n ? x[i].z : -INFINITY);
@@ -881,178 +847,267 @@ __global__ __launch_bounds__(kSmRows * 64) void k_attn_softmax_rows(attn_rows_ar
         }
     }
     mx = wm_wave_max_nonan(mx);
-    if (!isfinite(mx)) {  // every weight becomes 0 (or the row held a NaN)
-        for (uint32_t k = lane; k < n; k += 64) w[k] = 0.0f;
-        if (lane < n_tiles) live[lane] = 0;
-        if (lane == 0) a.row_scale[row] = 0.0f;
-        return;
-    }
-    // steps of 512: lane l takes positions k + 8l .. k + 8l + 7; the next
-    // step's scores are loaded before this step's sum
-    float4 c0 = w4[min(2 * lane, n4 - 1)], c1 = w4[min(2 * lane + 1, n4 - 1)];
-    float sum = 0.0f;
-    for (uint32_t k = 0; k < n; k += wm::kSeqBatch) {
-        const uint32_t base = k + 8 * lane;
-        float4 n0 = c0, n1 = c1;
-        if (k + wm::kSeqBatch < n) {
-            const uint32_t nq = (base + wm::kSeqBatch) / 4;
-            n0 = w4[min(nq, n4 - 1)];
-            n1 = w4[min(nq + 1, n4 - 1)];
-        }
-        float v[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-        bool nz = false;
+    if (WPR > 1 && lane == 0) red[wid] = mx;
+    __syncthreads();
+    if (WPR > 1)
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            v[j] = base + j < n ? wm::expf_glibc(v[j] - mx, exp_tab) : 0.0f;
-            nz = nz || v[j] != 0.0f;
-        }
-        if (base + 8 <= n) {
-            *reinterpret_cast<float4 *>(w + base) = make_float4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<float4 *>(w + base + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        } else {
+        for (uint32_t i = 0; i < WPR; i++) mx = wm_max_nonan(mx, red[r * WPR + i]);
+    const bool zero = !isfinite(mx);  // every weight becomes 0 (or the row held a NaN)
+    float s = 0.0f;                   // wave 0: the sum of row lane / 16
+    // this wave's part of chunk c: exps in place and into LDS (zeros past a
+    // shorter row's end change nothing)
+    const auto exps = [&](uint32_t c) {
 #pragma unroll
-            for (int j = 0; j < 8; j++)
-                if (base + j < n) w[base + j] = v[j];
+        for (uint32_t u = 0; u < kMine; u++) {
+            const uint32_t i = c * kMine + u, k = i * WPR + part;
+            float4 e = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (i < F4 && 256 * k < n) {
+                const uint32_t p = 256 * k + 4 * lane;
+                float4 &v = x[i < F4 ? i : 0];
+                if (!zero) {
+                    e.x = p < n ? exp_nonpos(v.x - mx, exp_tab) : 0.0f;
+                    e.y = p + 1 < n ? exp_nonpos(v.y - mx, exp_tab) : 0.0f;
+                    e.z = p + 2 < n ? exp_nonpos(v.z - mx, exp_tab) : 0.0f;
+                    e.w = p + 3 < n ? exp_nonpos(v.w - mx, exp_tab) : 0.0f;
+                }
+                v = e;
+                // lanes 16 j .. 16 j + 15 hold tile 4 k + j
+                const uint64_t nz = __ballot(e.x != 0.0f || e.y != 0.0f || e.z != 0.0f || e.w != 0.0f);
+                if (mine && lane < 4 && (4 * k + lane) * kSvPos < n)
+                    a.live[(uint64_t)row * kAttnTiles + 4 * k + lane] = (nz >> (16 * lane) & 0xFFFFu) != 0 ? 1 : 0;
+            }
+            *reinterpret_cast<float4 *>(&buf[c % kBufs][r][256 * (k % kSlots) + 4 * lane]) = e;
         }
-        // lanes 8i .. 8i+7 hold tile k / kSvPos + i
-        const uint64_t nzm = __ballot(nz);
-        const uint32_t tile = k / kSvPos + lane;
-        if (lane < 8 && tile < n_tiles) live[tile] = ((nzm >> (8 * lane)) & 0xFFu) != 0 ? 1 : 0;
-        sum = wm::seq_sum_step(sum, v, k == 0);
-        c0 = n0;
-        c1 = n1;
+    };
+    const auto chain = [&](uint32_t c) {
+        const float *src = buf[c % kBufs][lane / 16];
+        const uint32_t m = min(kSmChunk, n_max - c * kSmChunk);
+        // 32 terms per step, each half's reads ahead of the other's adds
+        float4 f[2][4];
+        const auto read16 = [&](float4 (&g)[4], uint32_t q) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) g[i] = *reinterpret_cast<const float4 *>(src + q + 4 * i);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        const auto add16 = [&](const float4 (&g)[4]) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) {
+                s = s + g[i].x;
+                s = s + g[i].y;
+                s = s + g[i].z;
+                s = s + g[i].w;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        read16(f[0], 0);
+        __builtin_amdgcn_s_setprio(3);  // (the chain's wave first on its SIMD: the others wait for it)
+#pragma unroll 1
+        for (uint32_t q = 0; q < m; q += 32) {
+            // (what a step adds past m is zeros; past the chunk nothing is read)
+            read16(f[1], q + 16);
+            add16(f[0]);
+            read16(f[0], q + 32 < kSmChunk ? q + 32 : 0u);
+            add16(f[1]);
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+    exps(0);
+#pragma unroll
+    for (uint32_t c = 0; c < kChunks; c++) {
+        if (c * kSmChunk >= n_max) break;
+        __syncthreads();  // chunk c is in LDS; chunk c - 1 is summed
+        if (c + 1 < kChunks && (c + 1) * kSmChunk < n_max) exps(c + 1);
+        if (wid == 0) chain(c);
     }
-    if (lane == 0) a.row_scale[row] = sum > 0.0f ? 1.0f / sum : 1.0f;
+    if (wid == 0 && lane % 16 == 0) row_inv[lane / 16] = s > 0.0f ? 1.0f / s : 1.0f;
+    __syncthreads();
+    if (!mine) return;
+    const float inv = row_inv[r];
+    const uint32_t end = (n + kSvPos - 1) / kSvPos * kSvPos;
+#pragma unroll
+    for (uint32_t i = 0; i < F4; i++) {
+        const uint32_t p = 256 * (i * WPR + part) + 4 * lane;
+        if (p < end)
+            *reinterpret_cast<float4 *>(w + p) = make_float4(x[i].x * inv, x[i].y * inv, x[i].z * inv, x[i].w * inv);
+    }
 }
 
-// One group of 8 positions of a staged tile, as thread d reads it: the V
-// codes vt[q][d], the rows' scales and the C chains' weights.
-template <uint32_t C>
-struct sv_group {
-    int code[8];
-    float4 sc[2];
-    float4 w[C][2];
-};
-template <int HD, uint32_t C>
-__device__ __forceinline__ void sv_read(sv_group<C> &g, const int8_t (*vt)[HD], const float *vst,
-                                        const float (*wt)[kSvPos], uint32_t q0) {
-#pragma unroll
-    for (uint32_t j = 0; j < 8; j++) g.code[j] = vt[q0 + j][threadIdx.x];
-    g.sc[0] = *reinterpret_cast<const float4 *>(&vst[q0]);
-    g.sc[1] = *reinterpret_cast<const float4 *>(&vst[q0 + 4]);
-#pragma unroll
-    for (uint32_t c = 0; c < C; c++) {
-        g.w[c][0] = *reinterpret_cast<const float4 *>(&wt[c][q0]);
-        g.w[c][1] = *reinterpret_cast<const float4 *>(&wt[c][q0 + 4]);
-    }
-}
-// acc[c] += w * v for the group's positions in order (v = q8 * scale: read_into)
-template <uint32_t C>
-__device__ __forceinline__ void sv_sum(float (&acc)[C], const sv_group<C> &g) {
-    const float sc[8] = {g.sc[0].x, g.sc[0].y, g.sc[0].z, g.sc[0].w, g.sc[1].x, g.sc[1].y, g.sc[1].z, g.sc[1].w};
-    float v[8];
-#pragma unroll
-    for (uint32_t j = 0; j < 8; j++) v[j] = (float)g.code[j] * sc[j];
-#pragma unroll
-    for (uint32_t c = 0; c < C; c++) {
-        const float w[8] = {g.w[c][0].x, g.w[c][0].y, g.w[c][0].z, g.w[c][0].w,
-                            g.w[c][1].x, g.w[c][1].y, g.w[c][1].z, g.w[c][1].w};
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) acc[c] = acc[c] + w[j] * v[j];
-    }
+// One wave's LDS operations complete in order; the compiler keeps that order
+// across this point.
+__device__ __forceinline__ void wave_lds_order() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// G: query heads per workgroup, HG: per KV head (item unit = kv head * HG/G + part)
-template <int HD, int G, int HG>
-__global__ __launch_bounds__(HD) void k_attn_sv_rows(attn_rows_args a) {
-    constexpr uint32_t C = kSvTok * G;  // chains per thread: c = token * G + head
-    __shared__ __align__(16) int8_t vt[kSvPos][HD];
-    __shared__ __align__(16) float vst[kSvPos];
-    __shared__ __align__(16) float wt[C][kSvPos];
-    __shared__ uint64_t live_mask;
+// out[t][h][d] = Σ_p w_h[p] * v_p[d] in position order (cached_forward.rs:
+// 417-449; v_p[d] = q8 * scale, read_into), w the softmax's weights.  A wave
+// runs C query heads of one KV head for one token ("row set"), lane = one of
+// 64 dimensions, over the row set's live tiles (a tile dead for some of the
+// heads adds zeros to them): the heads share each dequantised value.  The
+// next tile's codes, weights and scales are in flight behind the one in use;
+// the weights and V scales, the same for every lane, go through LDS as
+// broadcasts, four positions per read, read ahead of use.
+// Bound by VALU issue, 2 C + 2 instructions per position, and by the longest
+// rows: a wave issues one instruction in ~4 cycles at best, so they go first
+// (item order, s_setprio).  Other ways to a weight: as a scalar operand the
+// load takes ~750 cycles, more than 32 scalars in flight cover (173-181 us at
+// the ragged shape below); as a DPP broadcast the multiply issues at 0.4 of
+// its rate; a readlane takes three slots; products from a 4 x 4 x 1 MFMA
+// (exact, four rows at once) took 178.  The kernel it replaces ran one head per
+// workgroup, a byte read from LDS per position and lane.  Per BitNet-2B layer:
+// 512 prompt tokens 70 -> 36 us, 32 tokens at context 3000 74 -> 67, 16 ragged
+// sequences (293 tokens) 275 -> 159.
+template <int HD, int C>
+__global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t group) {
+    constexpr uint32_t NH = HD / 64;  // waves per row set
+    constexpr uint32_t kDimRow = 20;  // dwords of a dimension's 64 codes in LDS (spread banks)
+    __shared__ __align__(16) uint32_t lds[4][64 * kDimRow];
+    __shared__ __align__(16) float wts[4][C + 1][kSvPos];  // the tile's weights, V scales
     const wm_attn_item it = a.sv_items[blockIdx.x];
-    if (it.nt == 0) return;
-    const uint32_t kvh = it.unit / (HG / G), h0 = it.unit * G;  // first query head
-    const uint32_t tid = threadIdx.x;
-    const wm_batch_tok tk = a.tok[it.t0];  // the item's tokens share this cache
-    const uint32_t n = it.p1;              // the last token's context: every tile any chain needs
-    uint32_t nt_ctx[kSvTok];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (wid / NH >= it.nt) return;
+    const uint32_t rs = it.p0 + wid / NH, per = group / C;  // row set, row sets per token
+    const uint32_t t = it.t0 + rs / per, h0 = it.unit * group + rs % per * C;
+    const wm_batch_tok tk = a.tok[t];
+    const uint32_t n = tk.pos + 1;
+    const uint64_t row = (uint64_t)t * a.n_heads + h0;
+    // the tiles where any of the heads has a non-zero weight
+    bool lv = false;
+    if (lane * kSvPos < n)
 #pragma unroll
-    for (uint32_t tt = 0; tt < kSvTok; tt++) nt_ctx[tt] = tt < it.nt ? a.tok[it.t0 + tt].pos + 1 : 0u;
-    // the tiles where any chain has a non-zero exp, in position order
-    const uint32_t n_tiles = (n + kSvPos - 1) / kSvPos;
-    if (tid < 64) {
-        bool lv = false;
-        if (tid < n_tiles)
-#pragma unroll
-            for (uint32_t c = 0; c < C; c++)
-                if (c / G < it.nt && tid * kSvPos < nt_ctx[c / G])
-                    lv = lv || a.live[((uint64_t)(it.t0 + c / G) * a.n_heads + h0 + c % G) * kAttnTiles + tid];
-        const uint64_t mask = __ballot(lv);
-        if (tid == 0) live_mask = mask;
-    }
+        for (uint32_t c = 0; c < (uint32_t)C; c++) lv = lv || a.live[(row + c) * kAttnTiles + lane];
+    uint64_t mask = __ballot(lv);
     const uint64_t lay = (uint64_t)a.layer * tk.max_seq;
-    const int8_t *vg = tk.v + lay * a.kv_dim + kvh * HD;
-    const float *vsg = tk.vs + lay;
+    const uint32_t d0 = (wid % NH) * 64;
+    const wm_global_i8 *vg = (const wm_global_i8 *)tk.v + lay * a.kv_dim + it.unit * HD + d0;
+    const wm_global_f32 *vs = (const wm_global_f32 *)tk.vs + lay;
+    const wm_global_f32 *w0 = (const wm_global_f32 *)a.scores + row * a.score_stride;
     float acc[C];
 #pragma unroll
-    for (uint32_t c = 0; c < C; c++) acc[c] = 0.0f;
-    // this thread's weight slots e = tid + k * HD of a tile: chain e / kSvPos,
-    // position e % kSvPos; the row's exps and its 1/sum
-    constexpr uint32_t WK = (C * kSvPos + HD - 1) / HD;
-    const float *wrow[WK];
-    float wscale[WK];
-    uint32_t wlim[WK];
-#pragma unroll
-    for (uint32_t k = 0; k < WK; k++) {
-        const uint32_t e = min(tid + k * HD, C * kSvPos - 1), c = e / kSvPos, tt = c / G;
-        const uint64_t row = (uint64_t)(it.t0 + min(tt, it.nt - 1)) * a.n_heads + h0 + c % G;
-        wrow[k] = a.scores + row * a.score_stride + e % kSvPos;
-        wscale[k] = a.row_scale[row];
-        // positions below this one count (none for a slot past the tile)
-        wlim[k] = tt < it.nt && tid + k * HD < C * kSvPos ? nt_ctx[tt] : 0u;
-    }
-    float wr[WK];  // the next tile's exps, loaded with its V codes
-    const auto wfetch = [&](uint32_t p0) {
-#pragma unroll
-        for (uint32_t k = 0; k < WK; k++)
-            wr[k] = p0 + (tid + k * HD) % kSvPos < wlim[k] ? wrow[k][p0] : 0.0f;
+    for (int c = 0; c < C; c++) acc[c] = 0.0f;
+
+    // A tile as loaded.  Codes: lane 16 s + g takes dimensions 4 g .. 4 g+3 (a
+    // dword) of positions 16 i + 4 s + j, dword 4 i + j.  The
+    // heads' weights and the V scale of position `lane`.
+    // (Positions from n to the tile's end have zero weights.  Their codes and
+    // scales are whatever the cache holds there, always finite: it is
+    // allocated a tile longer and its scales start as zeros.)
+    struct tile_regs {
+        uint32_t v[16];
+        float x[C + 1];
     };
-    __syncthreads();
-    uint64_t mask = live_mask;
-    sv_regs pr{};
-    if (mask) {
-        sv_fetch<HD>(pr, vg, vsg, a.kv_dim, (uint32_t)__builtin_ctzll(mask) * kSvPos, n);
-        wfetch((uint32_t)__builtin_ctzll(mask) * kSvPos);
-    }
-    while (mask) {
+    uint32_t v_off[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) v_off[j] = (4 * (lane >> 4) + j) * a.kv_dim + 4 * (lane & 15);
+    const auto fetch = [&](tile_regs &q, uint32_t p) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            const wm_global_i8 *vp = vg + (uint64_t)(p + 16 * i) * a.kv_dim;
+            asm volatile("" : "+s"(vp));
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+                // (opaque: its widening stays at the load, which then takes a
+                // scalar base and this 32-bit offset)
+                asm volatile("" : "+v"(v_off[j]));
+                q.v[4 * i + j] = *(const uint32_t __attribute__((address_space(1))) *)(vp + v_off[j]);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < C; c++) q.x[c] = w0[(uint64_t)c * a.score_stride + p + lane];
+        q.x[C] = vs[p + lane];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Each dimension's 64 codes to its lane, through LDS: four positions'
+    // bytes of a dimension per dword (4 x 4 byte transposes), lane d reads
+    // slots s of dwords i: positions 16 i + 4 s ..  (A dimension's slots are
+    // XORed with its bits 5:4, so that eight lanes' accesses share no bank.)
+    uint32_t *const my = lds[wid];
+    const auto turn = [&](const tile_regs &q, uint32_t (&o)[16]) {
+#pragma unroll
+        for (int c = 0; c <= C; c++) wts[wid][c][lane] = q.x[c];
+        uint32_t td[4][4];  // [dimension][i]
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            const uint32_t x0 = q.v[4 * i], x1 = q.v[4 * i + 1], x2 = q.v[4 * i + 2], x3 = q.v[4 * i + 3];
+            const uint32_t a01 = __builtin_amdgcn_perm(x1, x0, 0x05010400u), b01 = __builtin_amdgcn_perm(x1, x0, 0x07030602u);
+            const uint32_t a23 = __builtin_amdgcn_perm(x3, x2, 0x05010400u), b23 = __builtin_amdgcn_perm(x3, x2, 0x07030602u);
+            td[0][i] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
+            td[1][i] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
+            td[2][i] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
+            td[3][i] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
+        }
+#pragma unroll
+        for (uint32_t d = 0; d < 4; d++)
+            *reinterpret_cast<uint4 *>(my + (4 * (lane & 15) + d) * kDimRow + 4 * ((lane >> 4) ^ ((lane >> 2) & 3))) =
+                make_uint4(td[d][0], td[d][1], td[d][2], td[d][3]);
+        wave_lds_order();
+#pragma unroll
+        for (uint32_t s = 0; s < 4; s++) {
+            const uint4 r = *reinterpret_cast<const uint4 *>(my + lane * kDimRow + 4 * (s ^ (lane >> 4)));
+            o[s] = r.x;  // dword 4 i + s: positions 16 i + 4 s .. + 3
+            o[4 + s] = r.y;
+            o[8 + s] = r.z;
+            o[12 + s] = r.w;
+        }
+        wave_lds_order();
+    };
+    constexpr uint32_t kL = C == 4 ? 4 : 8;  // positions read ahead
+    struct block {
+        float4 w[C][kL / 4], s[kL / 4];
+    };
+    const auto read = [&](block &q, uint32_t e) {
+#pragma unroll
+        for (uint32_t i = 0; i < kL / 4; i++) {
+            q.s[i] = *reinterpret_cast<const float4 *>(&wts[wid][C][e + 4 * i]);
+#pragma unroll
+            for (int c = 0; c < C; c++) q.w[c][i] = *reinterpret_cast<const float4 *>(&wts[wid][c][e + 4 * i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the reads go out before the terms that follow
+    };
+    const auto pick = [](const float4 &x, uint32_t e) { return e == 0 ? x.x : e == 1 ? x.y : e == 2 ? x.z : x.w; };
+    const auto add = [&](const block &q, const uint32_t (&v)[16], uint32_t e0) {
+#pragma unroll
+        for (uint32_t e = 0; e < kL; e++) {
+            const float f = (float)(int8_t)(v[(e0 + e) / 4] >> (8 * (e % 4))) * pick(q.s[e / 4], e % 4);  // read_into
+#pragma unroll
+            for (int c = 0; c < C; c++) acc[c] = acc[c] + pick(q.w[c][e / 4], e % 4) * f;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const auto next_tile = [&]() {
+        const uint32_t r = (uint32_t)__builtin_ctzll(mask) * kSvPos;
         mask &= mask - 1;
-        __syncthreads();  // the previous tile is summed
-        sv_stage<HD>(pr, vt, vst);
+        return r;
+    };
+    if (mask) {
+        // The longest rows end last: their waves go first on their SIMDs.
+        const uint32_t q = n * 4 / a.n_max;
+        if (q >= 3) __builtin_amdgcn_s_setprio(3);
+        else if (q == 2) __builtin_amdgcn_s_setprio(2);
+        else if (q == 1) __builtin_amdgcn_s_setprio(1);
+        tile_regs cur;
+        uint32_t v[16];
+        block qa, qb;
+        fetch(cur, next_tile());
+        for (bool more = true; more;) {
+            turn(cur, v);
+            read(qa, 0);
+            more = mask != 0;
+            if (more) fetch(cur, next_tile());
 #pragma unroll
-        for (uint32_t k = 0; k < WK; k++)
-            if (tid + k * HD < C * kSvPos) (&wt[0][0])[tid + k * HD] = wr[k] * wscale[k];  // exp * (1/sum)
-        __syncthreads();
-        if (mask) {
-            sv_fetch<HD>(pr, vg, vsg, a.kv_dim, (uint32_t)__builtin_ctzll(mask) * kSvPos, n);
-            wfetch((uint32_t)__builtin_ctzll(mask) * kSvPos);
-        }
-        // groups of 8 positions; a group's LDS reads are issued before the
-        // previous group is summed, so their latency overlaps that work
-        sv_group<C> ga, gb;
-        sv_read<HD, C>(ga, vt, vst, wt, 0);
-#pragma unroll
-        for (uint32_t q = 0; q < kSvPos; q += 16) {
-            sv_read<HD, C>(gb, vt, vst, wt, q + 8);
-            sv_sum<C>(acc, ga);
-            if (q + 16 < kSvPos) sv_read<HD, C>(ga, vt, vst, wt, q + 16);
-            sv_sum<C>(acc, gb);
+            for (uint32_t e = 0; e < kSvPos; e += 2 * kL) {
+                read(qb, e + kL);
+                add(qa, v, e);
+                if (e + 2 * kL < kSvPos) read(qa, e + 2 * kL);
+                add(qb, v, e + kL);
+            }
+            wave_lds_order();  // the tile's weights are read
         }
     }
+    float *out = a.out + row * HD + d0 + lane;
 #pragma unroll
-    for (uint32_t c = 0; c < C; c++)
-        if (c / G < it.nt)
-            a.out[(uint64_t)(it.t0 + c / G) * a.n_heads * HD + (uint64_t)(h0 + c % G) * HD + tid] = acc[c];
+    for (int c = 0; c < C; c++) out[c * HD] = acc[c];
 }
 
 }  // namespace
@@ -1163,27 +1218,22 @@ bool wm_attn_rows_supported(uint32_t head_dim, uint32_t group) {
            (group == 1 || group == 2 || group == 4 || group == 8);
 }
 
-// scores [m][n_heads][stride] | row scales [m][n_heads] | live tiles [m][n_heads][kAttnTiles]
+// scores [m][n_heads][stride] (whole tiles) | live tiles [m][n_heads][kAttnTiles]
+static uint32_t attn_stride(uint32_t n_max) { return (n_max + kSvPos - 1) / kSvPos * kSvPos; }
 static size_t attn_scores_part(uint32_t m, uint32_t n_heads, uint32_t n_max) {
-    return ((size_t)m * n_heads * ((n_max + 3u) & ~3u) * sizeof(float) + 255) & ~(size_t)255;
-}
-static size_t attn_scale_part(uint32_t m, uint32_t n_heads) {
-    return ((size_t)m * n_heads * sizeof(float) + 255) & ~(size_t)255;
+    return ((size_t)m * n_heads * attn_stride(n_max) * sizeof(float) + 255) & ~(size_t)255;
 }
 static size_t attn_live_part(uint32_t m, uint32_t n_heads) {
     return ((size_t)m * n_heads * kAttnTiles + 255) & ~(size_t)255;
 }
 size_t wm_attn_rows_scores_bytes(uint32_t m, uint32_t n_heads, uint32_t n_max, uint32_t n_items) {
-    return attn_scores_part(m, n_heads, n_max) + attn_scale_part(m, n_heads) +
-           attn_live_part(m, n_heads) + (size_t)n_items * sizeof(wm_attn_item);
+    return attn_scores_part(m, n_heads, n_max) + attn_live_part(m, n_heads) + (size_t)n_items * sizeof(wm_attn_item);
 }
 wm_attn_item *wm_attn_rows_items(float *scores, uint32_t m, uint32_t n_heads, uint32_t n_max) {
     return reinterpret_cast<wm_attn_item *>(reinterpret_cast<uint8_t *>(scores) +
                                             attn_scores_part(m, n_heads, n_max) +
-                                            attn_scale_part(m, n_heads) + attn_live_part(m, n_heads));
+                                            attn_live_part(m, n_heads));
 }
-
-uint32_t wm_attn_rows_sv_parts(uint32_t group) { return group < kSvHeads ? 1u : group / kSvHeads; }
 
 // Workgroup i runs on XCD i % 8.  The items of one (sequence, unit) read the
 // same K or V rows, so they share an XCD's L2 while that leaves the XCDs
@@ -1229,8 +1279,8 @@ static void attn_place(const std::vector<wm_attn_item> &items, const std::vector
         for (size_t k = 0; k < lists[x].size(); k++) out[k * kXcds + x] = items[lists[x][k]];
 }
 
-void wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t sc_units, uint32_t sv_units,
-                       std::vector<wm_attn_item> &sc, std::vector<wm_attn_item> &sv) {
+uint32_t wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t n_kv_heads, uint32_t group,
+                           uint32_t head_dim, std::vector<wm_attn_item> &sc, std::vector<wm_attn_item> &sv) {
     // the sequences: tokens of one cache at consecutive positions
     std::vector<std::pair<uint32_t, uint32_t>> seqs;
     for (uint32_t t = 0; t < m;) {
@@ -1246,49 +1296,58 @@ void wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t sc_units, u
         uint64_t waves = 0;
         for (auto &q : seqs)
             for (uint32_t b = q.first; b < q.second; b += nt_max)
-                waves += (uint64_t)sc_units * (tok[std::min(b + nt_max, q.second) - 1].pos / 64 + 1);
+                waves += (uint64_t)n_kv_heads * (tok[std::min(b + nt_max, q.second) - 1].pos / 64 + 1);
         if (waves >= 3 * kAttnSimds) break;
     }
     std::vector<wm_attn_item> items;
     std::vector<uint64_t> work;
-    std::vector<uint32_t> group;
+    std::vector<uint32_t> gids;
     uint32_t gid = 0;
     for (auto &q : seqs)
-        for (uint32_t u = 0; u < sc_units; u++, gid++)
+        for (uint32_t u = 0; u < n_kv_heads; u++, gid++)
             for (uint32_t b = q.first; b < q.second; b += nt_max) {
                 const uint32_t nt = std::min(nt_max, q.second - b), p1 = tok[b + nt - 1].pos + 1;
                 for (uint32_t p0 = 0; p0 < p1; p0 += kScoreThreads) {
                     items.push_back({b, nt, p0, p1, u, 0});
                     work.push_back((uint64_t)nt * std::min<uint32_t>(kScoreThreads, p1 - p0));
-                    group.push_back(gid);
+                    gids.push_back(gid);
                 }
             }
-    attn_place(items, work, group, sc);
+    attn_place(items, work, gids, sc);
     items.clear();
     work.clear();
-    group.clear();
+    gids.clear();
+    // V kernel: the most query heads per wave that leave four waves per SIMD,
+    // else fewer down to one (16 ragged sequences: 178 us with four heads,
+    // 159 with two, 225 with one; 512 prompt tokens: 36, 42 and more)
+    uint32_t heads = std::min(4u, group);
+    while (heads > 1 && (uint64_t)m * n_kv_heads * (group / heads) * (head_dim / 64) < 4 * kAttnSimds) heads /= 2;
+    const uint32_t waves_set = head_dim / 64, per_item = 4 / waves_set;  // waves per row set; row sets per item
+    const uint32_t per = group / heads;  // row sets per token and KV head
     for (auto &q : seqs)
-        for (uint32_t u = 0; u < sv_units; u++, gid++)
-            for (uint32_t b = q.first; b < q.second; b += kSvTok) {
-                const uint32_t nt = std::min<uint32_t>(kSvTok, q.second - b), p1 = tok[b + nt - 1].pos + 1;
-                items.push_back({b, nt, 0, p1, u, 0});
+        for (uint32_t u = 0; u < n_kv_heads; u++, gid++) {
+            const uint32_t sets = (q.second - q.first) * per;
+            for (uint32_t r = 0; r < sets; r += per_item) {
+                const uint32_t nt = std::min(per_item, sets - r), p1 = tok[q.first + (r + nt - 1) / per].pos + 1;
+                items.push_back({q.first, nt, r, p1, u, 0});
                 work.push_back((uint64_t)nt * p1);
-                group.push_back(gid);
+                gids.push_back(gid);
             }
-    attn_place(items, work, group, sv);
+        }
+    attn_place(items, work, gids, sv);
+    return heads;
 }
 
 void wm_launch_attn_rows(const float *q, const wm_batch_tok *tok, uint32_t m, uint32_t n_max,
                          uint32_t layer, uint32_t n_kv_heads, uint32_t head_dim, uint32_t group,
                          float scale, float *scores, float *out, uint32_t n_sc, uint32_t n_sv,
-                         hipStream_t s) {
+                         uint32_t sv_heads, hipStream_t s) {
     const uint32_t n_heads = n_kv_heads * group;
     uint8_t *base = reinterpret_cast<uint8_t *>(scores);
-    float *row_scale = reinterpret_cast<float *>(base + attn_scores_part(m, n_heads, n_max));
-    uint8_t *live = base + attn_scores_part(m, n_heads, n_max) + attn_scale_part(m, n_heads);
+    uint8_t *live = base + attn_scores_part(m, n_heads, n_max);
     const wm_attn_item *items = wm_attn_rows_items(scores, m, n_heads, n_max);
     attn_rows_args a{q, tok, scores, out, layer, n_kv_heads * head_dim, n_heads,
-                     (n_max + 3u) & ~3u, n_max, scale, row_scale, live, items, items + n_sc};
+                     attn_stride(n_max), n_max, scale, live, items, items + n_sc};
     const dim3 sgrid(n_sc);
 #define WM_SCORES_CASE(HD, G)                                                                  \
     if (head_dim == HD && group == G)                                                          \
@@ -1296,13 +1355,22 @@ void wm_launch_attn_rows(const float *q, const wm_batch_tok *tok, uint32_t m, ui
     WM_SCORES_CASE(128, 1) WM_SCORES_CASE(128, 2) WM_SCORES_CASE(128, 4) WM_SCORES_CASE(128, 8)
     WM_SCORES_CASE(64, 1) WM_SCORES_CASE(64, 2) WM_SCORES_CASE(64, 4) WM_SCORES_CASE(64, 8)
 #undef WM_SCORES_CASE
-    hipLaunchKernelGGL(k_attn_softmax_rows, dim3((n_heads + kSmRows - 1) / kSmRows, m), dim3(kSmRows * 64),
-                       0, s, a);
-#define WM_SV_CASE(HD, G)                                                                      \
-    if (head_dim == HD && group == G)                                                          \
-        hipLaunchKernelGGL((k_attn_sv_rows<HD, (G < kSvHeads ? G : kSvHeads), G>),             \
-                           dim3(n_sv), dim3(HD), 0, s, a);
-    WM_SV_CASE(128, 1) WM_SV_CASE(128, 2) WM_SV_CASE(128, 4) WM_SV_CASE(128, 8)
-    WM_SV_CASE(64, 1) WM_SV_CASE(64, 2) WM_SV_CASE(64, 4) WM_SV_CASE(64, 8)
+    const uint32_t n_rows = m * n_heads;
+    // Waves per row: one where a batch has rows enough to fill the chip, four
+    // for few rows of more than 1024 positions (each CU then holds eight).
+    const uint32_t wpr = n_max <= 1024 || n_rows > 8 * kGemmCus ? 1 : 4;
+    const uint32_t f4 = (n_max + 256 * wpr - 1) / (256 * wpr);
+    const dim3 sm_grid((n_rows + kSmRows - 1) / kSmRows);
+#define WM_SM_CASE(W, F)                                                                       \
+    if (wpr == W && f4 <= F && f4 > F / 2)                                                     \
+        hipLaunchKernelGGL((k_attn_softmax_rows<W, F>), sm_grid, dim3(kSmRows * W * 64), 0, s, a, n_rows);
+    WM_SM_CASE(1, 1) WM_SM_CASE(1, 2) WM_SM_CASE(1, 4) WM_SM_CASE(1, 8) WM_SM_CASE(1, 16)
+    WM_SM_CASE(4, 2) WM_SM_CASE(4, 4)
+#undef WM_SM_CASE
+#define WM_SV_CASE(HD, C)                                                                      \
+    if (head_dim == HD && sv_heads == C)                                           \
+        hipLaunchKernelGGL((k_attn_sv_rows<HD, C>), dim3(n_sv), dim3(256), 0, s, a, group);
+    WM_SV_CASE(128, 1) WM_SV_CASE(128, 2) WM_SV_CASE(128, 4)
+    WM_SV_CASE(64, 1) WM_SV_CASE(64, 2) WM_SV_CASE(64, 4)
 #undef WM_SV_CASE
 }

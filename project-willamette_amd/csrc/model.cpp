@@ -487,8 +487,7 @@ wm_status batch_forward_dev(wm_model *m, wm_kv_cache *const *caches, uint32_t n_
     hipStream_t s = ctx->stream;
     WM_HIP(ctx, hipSetDevice(m->device));
     std::vector<wm_attn_item> sc_items, sv_items;
-    wm_attn_rows_plan(tok.data(), M, c.n_kv_heads, c.n_kv_heads * wm_attn_rows_sv_parts(group),
-                      sc_items, sv_items);
+    const uint32_t sv_heads = wm_attn_rows_plan(tok.data(), M, c.n_kv_heads, group, c.head_dim, sc_items, sv_items);
     const uint32_t n_sc = (uint32_t)sc_items.size(), n_sv = (uint32_t)sv_items.size();
     sc_items.insert(sc_items.end(), sv_items.begin(), sv_items.end());
     const size_t sc_bytes = wm_attn_rows_scores_bytes(M, c.n_heads, n_max, n_sc + n_sv);
@@ -525,7 +524,7 @@ wm_status batch_forward_dev(wm_model *m, wm_kv_cache *const *caches, uint32_t n_
         wm_launch_qkv_rows(m->b_yqkv, QKV, m->rope_cos, m->rope_sin, m->b_tok, M, l, E, KV,
                            c.head_dim, c.n_rot, m->b_q, s);
         wm_launch_attn_rows(m->b_q, m->b_tok, M, n_max, l, c.n_kv_heads, c.head_dim, group, scale,
-                            m->b_scores, m->b_attn, n_sc, n_sv, s);
+                            m->b_scores, m->b_attn, n_sc, n_sv, sv_heads, s);
         nr = wm_norm_rows{m->b_attn, E, nullptr, 0, nullptr, 0, L.attn_sub_norm, E, c.rms_eps,
                           m->b_act, m_pad, m->b_meta, nullptr, 0, nullptr, 0};
         if (!wm_launch_rmsnorm_rows(nr, M, s)) return rows_unsupported(ctx);
@@ -791,10 +790,15 @@ wm_status wm_kv_cache_create(wm_model *m, uint32_t max_seq_len, wm_kv_cache **ou
     kv->max_seq = max_seq_len;
     const size_t nq = (size_t)m->cfg.n_layers * max_seq_len * m->kv_dim;
     const size_t ns = (size_t)m->cfg.n_layers * max_seq_len;
+    // V a tile longer, its scales from zeros: the batch's V pass reads whole
+    // tiles, with weight zero past a token's own position, and the scales
+    // there must be finite (any stored one is)
+    const size_t vs_bytes = (ns + WM_ATTN_TILE) * 4;
     hipError_t e = hipMalloc((void **)&kv->k, nq);
-    if (e == hipSuccess) e = hipMalloc((void **)&kv->v, nq);
+    if (e == hipSuccess) e = hipMalloc((void **)&kv->v, nq + (size_t)WM_ATTN_TILE * m->kv_dim);
     if (e == hipSuccess) e = hipMalloc((void **)&kv->ks, ns * 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&kv->vs, ns * 4);
+    if (e == hipSuccess) e = hipMalloc((void **)&kv->vs, vs_bytes);
+    if (e == hipSuccess) e = hipMemsetAsync(kv->vs, 0, vs_bytes, ctx->stream);
     if (e != hipSuccess) {
         wm_kv_cache_destroy(kv);
         return wm_hip_error(ctx, e, "KVCache::new");

@@ -33,28 +33,14 @@ constexpr uint64_t kExp2Tab[32] = {
     0x3fef5818dcfba487ull, 0x3fef7c97337b9b5full, 0x3fefa4afa2a490daull, 0x3fefd0765b6e4540ull,
 };
 
-// `tab` is kExp2Tab or a copy of it (device code passes an LDS copy so the
-// per-lane table lookup does not wait on global memory).
-WM_HD inline float expf_glibc(float x, const uint64_t *tab = kExp2Tab) {
+// The evaluation itself, for x of |x| < 88 and for larger ones down to
+// -0x1.9fe368p6 (a NaN stays one).
+WM_HD inline float expf_glibc_core(float x, const uint64_t *tab) {
     const double kInvLn2N = 0x1.71547652b82fep+0 * 32.0;
     const double kShift = 0x1.8p+52;
     const double kC0 = 0x1.c6af84b912394p-5 / (32.0 * 32.0 * 32.0);
     const double kC1 = 0x1.ebfce50fac4f3p-3 / (32.0 * 32.0);
     const double kC2 = 0x1.62e42ff0c52d6p-1 / 32.0;
-    uint32_t ux;
-    std::memcpy(&ux, &x, 4);
-    const uint32_t abstop = (ux >> 20) & 0x7ffu;
-    if (abstop >= 0x42bu) {  // |x| >= 88 or NaN
-        if (ux == 0xff800000u) return 0.0f;
-        if (abstop >= 0x7f8u) return x + x;
-        if (x > 0x1.62e42ep6f) {
-            const uint32_t inf = 0x7f800000u;
-            float r;
-            std::memcpy(&r, &inf, 4);
-            return r;
-        }
-        if (x < -0x1.9fe368p6f) return 0.0f;
-    }
     const double xd = (double)x;
     double kd = __builtin_fma(kInvLn2N, xd, kShift);
     uint64_t ki;
@@ -70,6 +56,26 @@ WM_HD inline float expf_glibc(float x, const uint64_t *tab = kExp2Tab) {
     y = __builtin_fma(z, r2, y);
     y = y * s;
     return (float)y;
+}
+
+// `tab` is kExp2Tab or a copy of it (device code passes an LDS copy so the
+// per-lane table lookup does not wait on global memory).
+WM_HD inline float expf_glibc(float x, const uint64_t *tab = kExp2Tab) {
+    uint32_t ux;
+    std::memcpy(&ux, &x, 4);
+    const uint32_t abstop = (ux >> 20) & 0x7ffu;
+    if (abstop >= 0x42bu) {  // |x| >= 88 or NaN
+        if (ux == 0xff800000u) return 0.0f;
+        if (abstop >= 0x7f8u) return x + x;
+        if (x > 0x1.62e42ep6f) {
+            const uint32_t inf = 0x7f800000u;
+            float r;
+            std::memcpy(&r, &inf, 4);
+            return r;
+        }
+        if (x < -0x1.9fe368p6f) return 0.0f;
+    }
+    return expf_glibc_core(x, tab);
 }
 
 }  // namespace wm

@@ -562,26 +562,29 @@ void wm_launch_qkv_rows(const float *y, uint32_t ldy, const float *rope_cos, con
                         hipStream_t s);
 // Causal GQA attention of every token of a batch over its own sequence cache.
 bool wm_attn_rows_supported(uint32_t head_dim, uint32_t group);
-// Work items of the batch attention, one per workgroup: tokens t0 .. t0+nt-1
-// of one sequence (nt = 0: nothing to do), positions [p0, p1) (scores) or
-// every position below p1 (V), KV head (scores) or KV-head part (V) `unit`.
+// Work items of the batch attention, one per workgroup (nt = 0: nothing to
+// do).  Scores: tokens t0 .. t0+nt-1 of one sequence, positions [p0, p1), KV
+// head `unit`.  V: of the sequence that starts at token t0, the row sets
+// p0 .. p0+nt-1 (a row set: some query heads of KV head `unit` for one token,
+// in token order), every position below p1.
 struct wm_attn_item {
     uint32_t t0, nt, p0, p1, unit, pad;
 };
 // From the step's tokens (host copy; a sequence's tokens are consecutive):
-// scores items per (sequence, KV head, up to 8 tokens, 256 positions) and V items
-// per (sequence, KV-head part, token), ordered so that the XCDs share the
-// work evenly and items that read the same rows share an XCD where they can.
-void wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t sc_units, uint32_t sv_units,
-                       std::vector<wm_attn_item> &sc, std::vector<wm_attn_item> &sv);
-// V-kernel units per KV head for a query group size
-uint32_t wm_attn_rows_sv_parts(uint32_t group);
-// Device workspace of one step: scores, row scales, live-tile flags and the
-// n_items work items (wm_attn_rows_items: where the items go).
+// scores items per (sequence, KV head, up to 8 tokens, 256 positions) and V
+// items per (sequence, KV head, a workgroup's row sets), ordered so that the
+// XCDs share the work evenly and items that read the same rows share an XCD
+// where they can.  Returns the query heads per V row set.
+uint32_t wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t n_kv_heads, uint32_t group,
+                           uint32_t head_dim, std::vector<wm_attn_item> &sc, std::vector<wm_attn_item> &sv);
+// The V kernel reads a tile of this many positions past a cache's last one.
+constexpr uint32_t WM_ATTN_TILE = 64;
+// Device workspace of one step: scores, live-tile flags and the n_items work
+// items (wm_attn_rows_items: where the items go).
 size_t wm_attn_rows_scores_bytes(uint32_t m, uint32_t n_heads, uint32_t n_max, uint32_t n_items);
 wm_attn_item *wm_attn_rows_items(float *scores, uint32_t m, uint32_t n_heads, uint32_t n_max);
 void wm_launch_attn_rows(const float *q, const wm_batch_tok *tok, uint32_t m, uint32_t n_max,
                          uint32_t layer, uint32_t n_kv_heads, uint32_t head_dim, uint32_t group,
                          float scale, float *scores, float *out, uint32_t n_sc, uint32_t n_sv,
-                         hipStream_t s);
+                         uint32_t sv_heads, hipStream_t s);
 void wm_launch_debug_seq_sum(const float *a, uint32_t n, float *out, hipStream_t s);

@@ -163,6 +163,49 @@ def test_batch_dense_softmax_long_rows(ctx):
     orm.close()
 
 
+@pytest.mark.parametrize("head_dim,group,n_kv,ctx_len,n_new,dense", [
+    # (rows' ends at 256, 512, 1024 and 2048 positions: the softmax's sizes;
+    # group and tokens: query heads and rows per wave of scores and V)
+    (64, 1, 4, 0, 3, True),
+    (64, 8, 1, 250, 9, True),
+    (64, 2, 2, 505, 11, True),
+    (128, 2, 1, 1020, 7, True),
+    (128, 8, 1, 2043, 8, False),
+    (128, 1, 4, 4070, 26, True),       # the last tile reaches past the context
+    (128, 4, 2, 63, 129, True),
+    (128, 4, 4, 0, 512, True),         # four heads per wave of V
+    (64, 4, 4, 1000, 300, False),      # two
+])
+def test_batch_attention_sizes_match_decode(ctx, head_dim, group, n_kv, ctx_len, n_new, dense):
+    """One sequence's tokens in a batch against the same tokens decoded one at
+    a time (checked against the oracle elsewhere): hidden state and cache
+    bytes, the second layer's of every token among them."""
+    n_embd = head_dim * group * n_kv
+    cfg = bs.BitNetConfig(n_layers=2, n_embd=n_embd, n_ff=384, n_heads=group * n_kv, n_kv_heads=n_kv,
+                          head_dim=head_dim, vocab=300, context_length=4096)
+    hm = bs.make_host_model(cfg, seed=head_dim + group)
+    if dense:  # scores so small that no weight underflows
+        for hl in hm.layers:
+            hl.scales["attn_q"] = 1e-6
+    dev = bs.load_device_model(ctx, hm)
+    rng = np.random.default_rng(ctx_len + n_new)
+    toks = rng.integers(0, cfg.vocab, n_new).tolist()
+    a, b = dev.kv_cache(4096), dev.kv_cache(4096)
+    if ctx_len:
+        k, v = bs.kv_prefill(cfg, seed=9, n_pos=ctx_len)
+        a.append_positions(k, v)
+        b.append_positions(k, v)
+    hidden, _ = dev.batch_forward([a], [toks])
+    for t in toks:
+        hb = b.forward(t, b.position)
+    assert bits_equal(hidden[0], hb)
+    for l in range(cfg.n_layers):
+        assert all(np.array_equal(x, y) for x, y in zip(a.read_raw(l, a.position), b.read_raw(l, b.position)))
+    a.close()
+    b.close()
+    dev.close()
+
+
 def test_batch_over_64_tokens(pair):
     # more than one 64-token GEMM tile, tiles shared by several sequences
     cfg, hm, dev, orm = pair
