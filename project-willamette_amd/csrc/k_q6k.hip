@@ -51,6 +51,7 @@
 namespace {
 
 constexpr int kLogitsBlock = 256;  // 4 waves
+constexpr int kFinalThreads = 512; // the candidates' maximum (one load per thread or two)
 constexpr int kMaxArgBlocks = 2048;
 constexpr int kBoundedBlock = 256;
 constexpr uint32_t kBoundedMaxBlocks = 2048;
@@ -319,6 +320,43 @@ __device__ __forceinline__ void q6_exact_accum(const q6_lane_blocks<CH> &v, uint
     }
 }
 
+// Whether one of the lane's d values is infinite or NaN.
+template <int CH>
+__device__ __forceinline__ bool q6_d_special(const q6_lane_blocks<CH> &v) {
+    bool sp = false;
+#pragma unroll
+    for (int j = 0; j < CH; j++) sp = sp || (q6_d_bits(v, j) & 0x7C00u) == 0x7C00u;
+    return sp;
+}
+// q6_exact_accum for a batch whose d values are all finite (the hardware's
+// f16 conversion is exact), with no path for the others beside it: that path
+// kept the registers of both alive.
+template <int CH>
+__device__ __forceinline__ void q6_exact_accum_finite(const q6_lane_blocks<CH> &v, const float *xb, float &acc) {
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+        uint32_t U[4];
+        q6_unpack(v.w0[j], v.w1[j], v.w2[j], U);
+        // (opaque, so that each quant is converted from its byte of U: seen
+        // through, the masks become a bit-field extract per quant)
+        asm volatile("" : "+v"(U[0]), "+v"(U[1]), "+v"(U[2]), "+v"(U[3]));
+        const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)q6_d_bits(v, j));
+#pragma unroll
+        for (int hn = 0; hn < 4; hn++) {
+            const float S = d * (float)(int)(int8_t)(v.scw[j] >> (8 * hn));
+            const float nS32 = -32.0f * S;
+            const float4 x4 = *reinterpret_cast<const float4 *>(xb + j * 16 + hn * 4);
+            const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float qf = (float)((U[hn] >> (8 * c)) & 0xFFu);
+                const float qS = __builtin_fmaf(qf, S, nS32);  // exact, as above
+                acc = acc + qS * xv[c];
+            }
+        }
+    }
+}
+
 // Combine the 16 partials of a lane group: v_l = (p0l + p1l) + (p2l + p3l);
 // dot = (v0 + v3) + (v1 + v2).  The dot ends up in all 16 lanes.
 __device__ __forceinline__ float q6_combine(float acc) {
@@ -328,13 +366,20 @@ __device__ __forceinline__ float q6_combine(float acc) {
     return u + __shfl_xor(u, 1, 64);
 }
 
+// Each wave takes a contiguous run of row groups, batches of CH blocks at a
+// time, with batch t + 1's loads in flight while batch t is summed (two
+// register sets in turn).  Bound by VALU issue (4 instructions per weight for
+// the exact order: convert, scale, multiply, add; ~1.5 for unpacking and
+// scales) beside the 42 us a plain read of the table takes: 128256 x 2560
+// 72.5 -> 62.4 us (before: no batch in flight during the sums, a bit-field
+// extract per quant, and 5.2 row groups per wave, so a sixth round with a
+// fifth of the waves).  Three workgroups per CU: at four, 128 registers a
+// thread spill part of the second set (79 us).
 template <int CH>
-__global__ __launch_bounds__(kLogitsBlock) void k_q6k_logits(
+__global__ __launch_bounds__(kLogitsBlock, 3) void k_q6k_logits(
     const uint8_t *__restrict__ w, uint32_t n_blocks, uint32_t n_rows, uint32_t n_rowgroups,
     const float *__restrict__ hidden, float *__restrict__ logits, argcand *__restrict__ cands) {
-    extern __shared__ float xs[];  // [16][n_blocks*16 + 4]
-    build_xs(hidden, n_blocks, xs);
-    __syncthreads();
+    extern __shared__ __align__(16) float xs[];  // [16][n_blocks*16 + 4]
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane >> 4, L = lane & 15;
@@ -344,24 +389,59 @@ __global__ __launch_bounds__(kLogitsBlock) void k_q6k_logits(
     float best_v = -INFINITY;
     uint32_t best_i = 0xFFFFFFFFu;
     constexpr uint32_t kWaves = kLogitsBlock / 64;
-    const uint32_t waves_total = gridDim.x * kWaves;
-    for (uint32_t G = blockIdx.x * kWaves + wave; G < n_rowgroups; G += waves_total) {
-        const __amdgpu_buffer_rsrc_t rs = wm_rsrc(w + (uint64_t)G * group_bytes, group_bytes);
-        float acc = 0.0f;
-        for (uint32_t b0 = 0; b0 < n_blocks; b0 += CH) {
-            q6_lane_blocks<CH> v;
-            q6_load_uniform<CH>(v, rs, b0, o);
-            q6_exact_accum<CH>(v, b0, xl, acc);
+    const uint32_t waves = gridDim.x * kWaves, id = blockIdx.x * kWaves + wave;
+    const uint32_t g0 = (uint32_t)((uint64_t)id * n_rowgroups / waves);
+    const uint32_t g1 = (uint32_t)((uint64_t)(id + 1) * n_rowgroups / waves);
+    const uint32_t per_group = n_blocks / CH, total = (g1 - g0) * per_group;  // batches
+    // (a batch past the last: the last one again, not used)
+    uint32_t ln = 0, lg = g0, lb = 0;  // the next batch to load: number, group, first block
+    const auto load = [&](q6_lane_blocks<CH> &v) {
+        q6_load_uniform<CH>(v, wm_rsrc(w + (uint64_t)lg * group_bytes, group_bytes), lb, o);
+        if (++ln < total && (lb += CH) == n_blocks) {
+            lb = 0;
+            lg++;
         }
-        const float dot = q6_combine(acc);
-        const uint32_t row = G * Q6K_GROUP_ROWS + r;
-        if (L == 0 && row < n_rows) {
-            if (logits) logits[row] = dot;
-            if (cand_better(dot, row, best_v, best_i)) {
-                best_v = dot;
-                best_i = row;
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out before the sums that follow
+    };
+    float acc = 0.0f;
+    uint32_t G = g0, b0 = 0;
+    const auto sum = [&](const q6_lane_blocks<CH> &v) {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(q6_d_special(v)) == 0, 1)) {
+            q6_exact_accum_finite<CH>(v, xl + b0 * 16, acc);
+        } else {  // (loaded again, a block at a time)
+#pragma unroll 1
+            for (uint32_t j = 0; j < CH; j++) {
+                q6_lane_blocks<1> u;
+                q6_load_lane<1>(u, w + (uint64_t)G * group_bytes, b0 + j, o);
+                q6_exact_accum<1>(u, b0 + j, xl, acc);
             }
         }
+        b0 += CH;
+        if (b0 == n_blocks) {
+            const float dot = q6_combine(acc);
+            const uint32_t row = G * Q6K_GROUP_ROWS + r;
+            if (L == 0 && row < n_rows) {
+                if (logits) logits[row] = dot;
+                if (cand_better(dot, row, best_v, best_i)) {
+                    best_v = dot;
+                    best_i = row;
+                }
+            }
+            acc = 0.0f;
+            b0 = 0;
+            G++;
+        }
+    };
+    q6_lane_blocks<CH> va, vb;
+    if (total) load(va);
+    build_xs(hidden, n_blocks, xs);
+    __syncthreads();
+    for (uint32_t t = 0; t < total; t += 2) {
+        load(vb);
+        sum(va);
+        if (t + 1 == total) break;
+        load(va);
+        sum(vb);
     }
     // block-wide best candidate
     for (int o = 32; o > 0; o >>= 1) {
@@ -385,11 +465,11 @@ __global__ __launch_bounds__(kLogitsBlock) void k_q6k_logits(
 
 // Combine the per-block candidates; a NaN logit at index 0 wins, as the
 // reference's scan starts from logits[0] and NaN compares false.
-__global__ void k_argmax_final(const argcand *__restrict__ cands, uint32_t n_cands,
+__global__ __launch_bounds__(kFinalThreads) void k_argmax_final(const argcand *__restrict__ cands, uint32_t n_cands,
                                const float *__restrict__ first_logit, uint32_t *__restrict__ out) {
     float bv = -INFINITY;
     uint32_t bi = 0xFFFFFFFFu;
-    for (uint32_t i = threadIdx.x; i < n_cands; i += 64)
+    for (uint32_t i = threadIdx.x; i < n_cands; i += kFinalThreads)
         if (cand_better(cands[i].v, cands[i].i, bv, bi)) {
             bv = cands[i].v;
             bi = cands[i].i;
@@ -402,7 +482,15 @@ __global__ void k_argmax_final(const argcand *__restrict__ cands, uint32_t n_can
             bi = oi;
         }
     }
+    __shared__ argcand s_c[kFinalThreads / 64];
+    if ((threadIdx.x & 63) == 0) s_c[threadIdx.x >> 6] = argcand{bv, bi};
+    __syncthreads();
     if (threadIdx.x == 0) {
+        for (int i = 1; i < kFinalThreads / 64; i++)
+            if (cand_better(s_c[i].v, s_c[i].i, bv, bi)) {
+                bv = s_c[i].v;
+                bi = s_c[i].i;
+            }
         float f0 = *first_logit;
         // every row's value is -inf or NaN: the scan keeps index 0
         *out = (f0 != f0 || bi == 0xFFFFFFFFu) ? 0u : bi;
@@ -1238,7 +1326,7 @@ void wm_launch_q6k_logits_argmax(const uint8_t *w, uint32_t n_blocks, uint32_t n
                                  uint32_t n_rowgroups, const float *hidden, float *logits,
                                  uint32_t *argmax_out, void *work, hipStream_t s) {
     uint32_t blocks = (n_rowgroups + 3) / 4;
-    const uint32_t max_blocks = 256 * 6;  // 24 waves per CU
+    const uint32_t max_blocks = 256 * 3;  // resident at once: three per CU
     if (blocks > max_blocks) blocks = max_blocks;
     if (blocks == 0) blocks = 1;
     const size_t lds = sizeof(float) * 16 * (n_blocks * 16 + 4);
@@ -1254,7 +1342,7 @@ void wm_launch_q6k_logits_argmax(const uint8_t *w, uint32_t n_blocks, uint32_t n
     }
 #undef WM_LOGITS_CASE
     if (argmax_out)
-        hipLaunchKernelGGL(k_argmax_final, dim3(1), dim3(64), 0, s, cands, blocks, logits,
+        hipLaunchKernelGGL(k_argmax_final, dim3(1), dim3(kFinalThreads), 0, s, cands, blocks, logits,
                            argmax_out);
 }
 
