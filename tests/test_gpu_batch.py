@@ -55,6 +55,36 @@ def test_matmul_rows_equal_single_row_path(ctx, in_dim, out_dim, m):
     w.close()
 
 
+@pytest.mark.parametrize("in_dim,shift", [
+    (128, 0), (1024, 0), (8192, 0),       # one unit of 16 columns per thread, the last a full workgroup
+    (8320, 0), (16384, 0),                # two
+    (16512, 0), (32768, 0),               # four
+    (32896, 0),                           # more: the row read twice
+    (2560, 1), (128, 3),                  # rows not 16-byte aligned
+])
+def test_matmul_quantiser_sizes(ctx, in_dim, shift):
+    """The row quantiser at the row lengths and alignments where its kernels
+    change, with NaN, infinite and zero rows: every output equals the
+    single-row path's."""
+    out_dim, m = 65, 5
+    rng = np.random.default_rng(in_dim + shift)
+    packed = rng.integers(0, 256, out_dim * in_dim // 4, dtype=np.uint8)
+    x = (rng.standard_normal((m, in_dim)) * 3).astype(np.float32)
+    x[1] = 0.0
+    x[2, in_dim // 2] = np.nan
+    x[3, in_dim - 1] = np.inf
+    w = ctx.upload_i2s(packed, 0.75, in_dim, out_dim)
+    dx = ctx.to_device(np.concatenate([np.zeros(shift, np.float32), x.ravel()]))
+    dy = ctx.alloc(m * out_dim * 4)
+    ctx.check(wh.lib.wm_bitlinear_i2s_matmul_f32_dev(ctx.h, w.h, dx.ptr + 4 * shift, m, dy.ptr))
+    y = dy.to_host(np.float32).reshape(m, out_dim)
+    for r in range(m):
+        ry, _, _, _ = orc.bitlinear_i8(packed, np.float32(0.75), in_dim, out_dim, x[r])
+        assert bits_equal(y[r], ry) or (np.isnan(ry).all() and np.isnan(y[r]).all()), f"row {r}"
+    for b in (dx, dy, w):
+        b.close()
+
+
 def test_matmul_rejects_bad_lengths(ctx):
     rng = np.random.default_rng(5)
     w = ctx.upload_i2s(rng.integers(0, 256, 64 * 128 // 4, dtype=np.uint8), 1.0, 128, 64)
