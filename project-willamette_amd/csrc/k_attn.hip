@@ -112,6 +112,11 @@ __device__ __forceinline__ uint64_t ld_tagged(const uint64_t *p) {
 constexpr int kSvThreads = 1024;  // wave 0: the 16 chains; waves 1-15: products
 constexpr int kSvDims = 16;        // head dims per workgroup (one 16-byte V segment)
 constexpr int kSvTile = 240;       // positions per product tile
+// products per step of the adds: one wave's dependent adds take ~5 cycles each,
+// and a step's LDS reads (12 of 16 bytes) up to ~200, which 24 products did
+// not cover (~10 cycles a term)
+constexpr int kSvStep = 48;
+static_assert(kSvTile % kSvStep == 0, "whole steps per tile");
 constexpr int kSvStride = 244;     // floats per dim row of a product tile (16-byte rows)
 constexpr uint32_t kSvSerialSum = 64;  // longest exp list summed by one wave, one add at a time
 static_assert(kSvTile * (kSvDims / 4) == kSvThreads - 64, "one 4-dim unit per producer thread");
@@ -519,13 +524,11 @@ __global__ __launch_bounds__(kSvThreads) void k_attn_decode(const float *q, cons
                 ev[jj] = ((uint32_t)jj < mm && k0 + (uint32_t)jj < count) ? cval[k0 + jj] : 0.0f;
             sum = wm::seq_sum_block_owned<MAXM, kSvThreads>(ev, count, cval, &seq_scratch);
         }
-        if (sum > 0.0f) {
-            const float inv = 1.0f / sum;
-            for (uint32_t k = tid; k < count; k += kSvThreads) cval[k] = cval[k] * inv;
-        }
-        wm_sync_lds();
-        // products of tile t (waves 1-15) while wave 0 adds tile t - 1,
-        // over the compacted positions in order
+        const float inv = sum > 0.0f ? 1.0f / sum : 1.0f;
+        // products (exp * (1/sum)) * v of tile t (waves 1-15) while wave 0
+        // adds tile t - 1, over the compacted positions in order.  The last
+        // tile's are zeros up to a whole step of the adds, which change
+        // nothing (a sum that starts at +0 is never -0).
         const uint32_t n_tiles = (count + kSvTile - 1) / kSvTile;
         const uint32_t pt = tid - 64, dq = pt / kSvTile, pl = pt % kSvTile;  // producer unit
         float acc = 0.0f;
@@ -540,44 +543,43 @@ __global__ __launch_bounds__(kSvThreads) void k_attn_decode(const float *q, cons
                         const uint32_t p = cidx[k];
                         float *dst = prod + (t & 1) * (kSvDims * kSvStride) + dq * 4 * kSvStride + pl;
                         const uint32_t word = reinterpret_cast<const uint32_t *>(vq + p)[dq];
-                        const float w = cval[k], s = vsc[p];
+                        const float w = cval[k] * inv, s = vsc[p];
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
                             const float vd = (float)(int8_t)(word >> (8 * i)) * s;  // read_into: q * scale
                             dst[i * kSvStride] = w * vd;                             // w * v_h[d]
                         }
+                    } else if (k < (count + kSvStep - 1) / kSvStep * kSvStep) {
+                        float *dst = prod + (t & 1) * (kSvDims * kSvStride) + dq * 4 * kSvStride + pl;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) dst[i * kSvStride] = 0.0f;
                     }
                 }
             } else if (lane < kSvDims && t > 0) {
                 const float *src = prod + ((t - 1) & 1) * (kSvDims * kSvStride) + lane * kSvStride;
-                const uint32_t k0 = (t - 1) * kSvTile;
-                const uint32_t tn = count - k0 < (uint32_t)kSvTile ? count - k0 : (uint32_t)kSvTile;
-                if (tn == (uint32_t)kSvTile) {
-                    // 24 products per step, the next step's reads issued before this step's adds
-                    constexpr int kC = 6, kSteps = kSvTile / (4 * kC);
-                    float4 f[2][kC];
+                const uint32_t tn = min(count - (t - 1) * kSvTile, (uint32_t)kSvTile);
+                // kSvStep products per step, the next step's reads issued
+                // before this step's adds, into two buffers in turn
+                constexpr int kC = kSvStep / 4, kSteps = kSvTile / kSvStep;
+                float4 f[2][kC];
 #pragma unroll
-                    for (int i = 0; i < kC; i++) f[0][i] = *reinterpret_cast<const float4 *>(src + 4 * i);
+                for (int i = 0; i < kC; i++) f[0][i] = *reinterpret_cast<const float4 *>(src + 4 * i);
 #pragma unroll
-                    for (int c4 = 0; c4 < kSteps; c4++) {
-                        if (c4 + 1 < kSteps) {
+                for (int c4 = 0; c4 < kSteps; c4++) {
+                    if (c4 * kSvStep >= (int)tn) break;
+                    // (past the tile's products: a read that is not used)
+                    if (c4 + 1 < kSteps) {
 #pragma unroll
-                            for (int i = 0; i < kC; i++)
-                                f[(c4 + 1) & 1][i] = *reinterpret_cast<const float4 *>(src + (c4 + 1) * 4 * kC + 4 * i);
-                        }
-#pragma unroll
-                        for (int i = 0; i < kC; i++) {
-                            const float4 gg = f[c4 & 1][i];
-                            acc = acc + gg.x; acc = acc + gg.y; acc = acc + gg.z; acc = acc + gg.w;
-                        }
+                        for (int i = 0; i < kC; i++)
+                            f[(c4 + 1) & 1][i] = *reinterpret_cast<const float4 *>(src + (c4 + 1) * kSvStep + 4 * i);
                     }
-                } else {
-                    uint32_t q = 0;
-                    for (; q + 4 <= tn; q += 4) {
-                        const float4 gg = *reinterpret_cast<const float4 *>(src + q);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < kC; i++) {
+                        const float4 gg = f[c4 & 1][i];
                         acc = acc + gg.x; acc = acc + gg.y; acc = acc + gg.z; acc = acc + gg.w;
                     }
-                    for (; q < tn; q++) acc = acc + src[q];
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
             wm_sync_lds();
