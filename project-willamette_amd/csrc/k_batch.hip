@@ -840,6 +840,7 @@ __global__ __launch_bounds__(kScoreThreads, 2) void k_attn_scores_rows(attn_rows
 
 constexpr uint32_t kSvPos = WM_ATTN_TILE;  // positions per tile of the V pass
 constexpr uint32_t kAttnTiles = 64;  // tiles per row (contexts <= 4096)
+constexpr uint32_t kSvDimRow = 20;   // dwords of a dimension's 64 codes of a tile in LDS (spread banks)
 
 // Softmax of the scores rows in place (attention.rs:45-73): max, exp (glibc
 // expf), the exact sequential sum of the exps, and each weight exp * (1/sum)
@@ -1004,50 +1005,18 @@ __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// out[t][h][d] = Σ_p w_h[p] * v_p[d] in position order (cached_forward.rs:
-// 417-449; v_p[d] = q8 * scale, read_into), w the softmax's weights.  A wave
-// runs C query heads of one KV head for one token ("row set"), lane = one of
-// 64 dimensions, over the row set's live tiles (a tile dead for some of the
-// heads adds zeros to them): the heads share each dequantised value.  The
-// next tile's codes, weights and scales are in flight behind the one in use;
-// the weights and V scales, the same for every lane, go through LDS as
-// broadcasts, four positions per read, read ahead of use.
-// Bound by VALU issue, 2 C + 2 instructions per position, and by the longest
-// rows: a wave issues one instruction in ~4 cycles at best, so they go first
-// (item order, s_setprio).  Other ways to a weight: as a scalar operand the
-// load takes ~750 cycles, more than 32 scalars in flight cover (173-181 us at
-// the ragged shape below); as a DPP broadcast the multiply issues at 0.4 of
-// its rate; a readlane takes three slots; products from a 4 x 4 x 1 MFMA
-// (exact, four rows at once) took 178.  The kernel it replaces ran one head per
-// workgroup, a byte read from LDS per position and lane.  Per BitNet-2B layer:
-// 512 prompt tokens 70 -> 36 us, 32 tokens at context 3000 74 -> 67, 16 ragged
-// sequences (293 tokens) 275 -> 159.
-template <int HD, int C>
-__global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t group) {
-    constexpr uint32_t NH = HD / 64;  // waves per row set
-    constexpr uint32_t kDimRow = 20;  // dwords of a dimension's 64 codes in LDS (spread banks)
-    __shared__ __align__(16) uint32_t lds[4][64 * kDimRow];
-    __shared__ __align__(16) float wts[4][C + 1][kSvPos];  // the tile's weights, V scales
-    const wm_attn_item it = a.sv_items[blockIdx.x];
+// One wave's part of k_attn_sv_rows: out[h][d] for its 64 dimensions (lane =
+// one of them) of the heads of one token, C at a time: heads 0 .. C-1 over the
+// tiles of ms[0], the next C over those of ms[1], and so on for all N masks
+// (w, out: head 0's weights and outputs).  The next tile's codes, weights and
+// scales are in flight behind the one in use, across the heads' ends too; the
+// weights and V scales, the same for every lane, go through LDS (wts, my: the
+// wave's own) as broadcasts, four positions per read, read ahead of use.
+template <int HD, int C, int N>
+__device__ __forceinline__ void sv_heads(const attn_rows_args &a, const wm_global_i8 *vg, const wm_global_f32 *vs,
+                                         const wm_global_f32 *w, float *out, float (*wts)[kSvPos], uint32_t *my,
+                                         uint64_t (&ms)[N]) {
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (wid / NH >= it.nt) return;
-    const uint32_t rs = it.p0 + wid / NH, per = group / C;  // row set, row sets per token
-    const uint32_t t = it.t0 + rs / per, h0 = it.unit * group + rs % per * C;
-    const wm_batch_tok tk = a.tok[t];
-    const uint32_t n = tk.pos + 1;
-    const uint64_t row = (uint64_t)t * a.n_heads + h0;
-    // the tiles where any of the heads has a non-zero weight
-    bool lv = false;
-    if (lane * kSvPos < n)
-#pragma unroll
-        for (uint32_t c = 0; c < (uint32_t)C; c++) lv = lv || a.live[(row + c) * kAttnTiles + lane];
-    uint64_t mask = __ballot(lv);
-    const uint64_t lay = (uint64_t)a.layer * tk.max_seq;
-    const uint32_t d0 = (wid % NH) * 64;
-    const wm_global_i8 *vg = (const wm_global_i8 *)tk.v + lay * a.kv_dim + it.unit * HD + d0;
-    const wm_global_f32 *vs = (const wm_global_f32 *)tk.vs + lay;
-    const wm_global_f32 *w0 = (const wm_global_f32 *)a.scores + row * a.score_stride;
     float acc[C];
 #pragma unroll
     for (int c = 0; c < C; c++) acc[c] = 0.0f;
@@ -1065,7 +1034,7 @@ __global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t
     uint32_t v_off[4];
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) v_off[j] = (4 * (lane >> 4) + j) * a.kv_dim + 4 * (lane & 15);
-    const auto fetch = [&](tile_regs &q, uint32_t p) {
+    const auto fetch = [&](tile_regs &q, uint32_t h, uint32_t p) {
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) {
             const wm_global_i8 *vp = vg + (uint64_t)(p + 16 * i) * a.kv_dim;
@@ -1079,7 +1048,7 @@ __global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t
             }
         }
 #pragma unroll
-        for (int c = 0; c < C; c++) q.x[c] = w0[(uint64_t)c * a.score_stride + p + lane];
+        for (uint32_t c = 0; c < (uint32_t)C; c++) q.x[c] = w[(uint64_t)(h + c) * a.score_stride + p + lane];
         q.x[C] = vs[p + lane];
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -1087,10 +1056,9 @@ __global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t
     // bytes of a dimension per dword (4 x 4 byte transposes), lane d reads
     // slots s of dwords i: positions 16 i + 4 s ..  (A dimension's slots are
     // XORed with its bits 5:4, so that eight lanes' accesses share no bank.)
-    uint32_t *const my = lds[wid];
     const auto turn = [&](const tile_regs &q, uint32_t (&o)[16]) {
 #pragma unroll
-        for (int c = 0; c <= C; c++) wts[wid][c][lane] = q.x[c];
+        for (int c = 0; c <= C; c++) wts[c][lane] = q.x[c];
         uint32_t td[4][4];  // [dimension][i]
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) {
@@ -1104,12 +1072,12 @@ __global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t
         }
 #pragma unroll
         for (uint32_t d = 0; d < 4; d++)
-            *reinterpret_cast<uint4 *>(my + (4 * (lane & 15) + d) * kDimRow + 4 * ((lane >> 4) ^ ((lane >> 2) & 3))) =
+            *reinterpret_cast<uint4 *>(my + (4 * (lane & 15) + d) * kSvDimRow + 4 * ((lane >> 4) ^ ((lane >> 2) & 3))) =
                 make_uint4(td[d][0], td[d][1], td[d][2], td[d][3]);
         wave_lds_order();
 #pragma unroll
         for (uint32_t s = 0; s < 4; s++) {
-            const uint4 r = *reinterpret_cast<const uint4 *>(my + lane * kDimRow + 4 * (s ^ (lane >> 4)));
+            const uint4 r = *reinterpret_cast<const uint4 *>(my + lane * kSvDimRow + 4 * (s ^ (lane >> 4)));
             o[s] = r.x;  // dword 4 i + s: positions 16 i + 4 s .. + 3
             o[4 + s] = r.y;
             o[8 + s] = r.z;
@@ -1124,9 +1092,9 @@ __global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t
     const auto read = [&](block &q, uint32_t e) {
 #pragma unroll
         for (uint32_t i = 0; i < kL / 4; i++) {
-            q.s[i] = *reinterpret_cast<const float4 *>(&wts[wid][C][e + 4 * i]);
+            q.s[i] = *reinterpret_cast<const float4 *>(&wts[C][e + 4 * i]);
 #pragma unroll
-            for (int c = 0; c < C; c++) q.w[c][i] = *reinterpret_cast<const float4 *>(&wts[wid][c][e + 4 * i]);
+            for (int c = 0; c < C; c++) q.w[c][i] = *reinterpret_cast<const float4 *>(&wts[c][e + 4 * i]);
         }
         __builtin_amdgcn_sched_barrier(0);  // the reads go out before the terms that follow
     };
@@ -1140,26 +1108,54 @@ __global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t
         }
         __builtin_amdgcn_sched_barrier(0);
     };
+    const auto store = [&](uint32_t h) {
+#pragma unroll
+        for (uint32_t c = 0; c < (uint32_t)C; c++) {
+            out[(h + c) * HD + lane] = acc[c];
+            acc[c] = 0.0f;
+        }
+    };
+    const auto remain = [&]() {
+        uint64_t m = ms[0];
+#pragma unroll
+        for (int i = 1; i < N; i++) m |= ms[i];
+        return m != 0;
+    };
+    // the heads of the next tile: those without one are left out
+    uint32_t h_next = 0;
+    const auto next_head = [&]() {  // (a mask is not empty)
+#pragma unroll
+        for (int i = 1; i < N; i++)
+            if (ms[0] == 0) {
+#pragma unroll
+                for (int k = 1; k < N; k++) ms[k - 1] = ms[k];
+                ms[N - 1] = 0;
+                h_next += C;
+            }
+    };
     const auto next_tile = [&]() {
-        const uint32_t r = (uint32_t)__builtin_ctzll(mask) * kSvPos;
-        mask &= mask - 1;
+        const uint32_t r = (uint32_t)__builtin_ctzll(ms[0]) * kSvPos;
+        ms[0] &= ms[0] - 1;
         return r;
     };
-    if (mask) {
-        // The longest rows end last: their waves go first on their SIMDs.
-        const uint32_t q = n * 4 / a.n_max;
-        if (q >= 3) __builtin_amdgcn_s_setprio(3);
-        else if (q == 2) __builtin_amdgcn_s_setprio(2);
-        else if (q == 1) __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (uint32_t i = 0; N > 1 && i < (uint32_t)N; i++)
+        if (ms[i] == 0) store(i * C);
+    if (remain()) {
         tile_regs cur;
         uint32_t v[16];
         block qa, qb;
-        fetch(cur, next_tile());
+        next_head();
+        uint32_t h = h_next;  // the heads of the tile in use
+        fetch(cur, h, next_tile());
         for (bool more = true; more;) {
             turn(cur, v);
             read(qa, 0);
-            more = mask != 0;
-            if (more) fetch(cur, next_tile());
+            more = remain();
+            if (more) {
+                next_head();
+                fetch(cur, h_next, next_tile());
+            }
 #pragma unroll
             for (uint32_t e = 0; e < kSvPos; e += 2 * kL) {
                 read(qb, e + kL);
@@ -1168,11 +1164,80 @@ __global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t
                 add(qb, v, e + kL);
             }
             wave_lds_order();  // the tile's weights are read
+            if (N > 1 && (!more || h_next != h)) {
+                store(h);
+                h = h_next;
+            }
         }
     }
-    float *out = a.out + row * HD + d0 + lane;
+    if (N == 1) store(0);
+}
+
+// out[t][h][d] = Σ_p w_h[p] * v_p[d] in position order (cached_forward.rs:
+// 417-449; v_p[d] = q8 * scale, read_into), w the softmax's weights.  A wave
+// runs C query heads of one KV head for one token ("row set"), lane = one of
+// 64 dimensions, over the row set's live tiles: together, the heads sharing
+// each dequantised value (a tile dead for some of them adds zeros to those),
+// or, where their live tiles are mostly different ones, one head after the
+// other, each over its own.
+// Bound by VALU issue, 2 C + 2 instructions per position, and by the longest
+// rows: a wave issues one instruction in ~4 cycles at best, so they go first
+// (item order, s_setprio).  Other ways to a weight: as a scalar operand the
+// load takes ~750 cycles, more than 32 scalars in flight cover (173-181 us at
+// the ragged shape below); as a DPP broadcast the multiply issues at 0.4 of
+// its rate; a readlane takes three slots; products from a 4 x 4 x 1 MFMA
+// (exact, four rows at once) took 178.  The kernel it replaces ran one head per
+// workgroup, a byte read from LDS per position and lane.  Per BitNet-2B layer:
+// 512 prompt tokens 70 -> 36 us, 32 tokens at context 3000 74 -> 67, 16 ragged
+// sequences (293 tokens) 275 -> 159.  Where the softmaxes are sparse (16 ragged
+// sequences, 257 tokens, N(0,1) K and V: most rows one live tile, some all) a
+// wave over its heads' tiles together took 99 us, the kernel before it 90, one
+// head after the other where that is shorter 87; the choice costs dense rows
+// under 1 % (36, 68 and 157 us at the shapes above).
+template <int HD, int C>
+__global__ __launch_bounds__(256) void k_attn_sv_rows(attn_rows_args a, uint32_t group) {
+    constexpr uint32_t NH = HD / 64;  // waves per row set
+    __shared__ __align__(16) uint32_t lds[4][64 * kSvDimRow];
+    __shared__ __align__(16) float wts[4][C + 1][kSvPos];  // the tile's weights, V scales
+    const wm_attn_item it = a.sv_items[blockIdx.x];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (wid / NH >= it.nt) return;
+    const uint32_t rs = it.p0 + wid / NH, per = group / C;  // row set, row sets per token
+    const uint32_t t = it.t0 + rs / per, h0 = it.unit * group + rs % per * C;
+    const wm_batch_tok tk = a.tok[t];
+    const uint32_t n = tk.pos + 1;
+    const uint64_t row = (uint64_t)t * a.n_heads + h0;
+    // the tiles where each head, and where any of them, has a non-zero weight
+    uint32_t lv[C];
 #pragma unroll
-    for (int c = 0; c < C; c++) out[c * HD] = acc[c];
+    for (uint32_t c = 0; c < (uint32_t)C; c++)
+        lv[c] = a.live[(row + c) * kAttnTiles + min(lane, (n - 1) / kSvPos)];
+    const uint32_t in = lane * kSvPos < n ? 1u : 0u;
+    uint64_t own[C], any[1] = {0};
+    uint32_t tiles = 0;
+#pragma unroll
+    for (uint32_t c = 0; c < (uint32_t)C; c++) {
+        own[c] = __ballot((lv[c] & in) != 0);
+        any[0] |= own[c];
+        tiles += (uint32_t)__builtin_popcountll(own[c]);
+    }
+    const uint32_t shared = (uint32_t)__builtin_popcountll(any[0]);
+    const uint64_t lay = (uint64_t)a.layer * tk.max_seq;
+    const uint32_t d0 = (wid % NH) * 64;
+    const wm_global_i8 *vg = (const wm_global_i8 *)tk.v + lay * a.kv_dim + it.unit * HD + d0;
+    const wm_global_f32 *vs = (const wm_global_f32 *)tk.vs + lay;
+    const wm_global_f32 *w = (const wm_global_f32 *)a.scores + row * a.score_stride;
+    float *out = a.out + row * HD + d0;
+    // The longest rows end last: their waves go first on their SIMDs.
+    const uint32_t q = n * 4 / a.n_max;
+    if (q >= 3) __builtin_amdgcn_s_setprio(3);
+    else if (q == 2) __builtin_amdgcn_s_setprio(2);
+    else if (q == 1) __builtin_amdgcn_s_setprio(1);
+    // By the instructions of a tile: about C + 2 units with C heads at once, 3
+    // with one (~100 for the tile's codes and 64 (2 C + 2) + 17 (C + 1)).
+    if (C > 1 && tiles * 3 < shared * (C + 2)) sv_heads<HD, 1, C>(a, vg, vs, w, out, wts[wid], lds[wid], own);
+    else sv_heads<HD, C, 1>(a, vg, vs, w, out, wts[wid], lds[wid], any);
 }
 
 }  // namespace

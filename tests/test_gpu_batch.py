@@ -236,6 +236,40 @@ def test_batch_attention_sizes_match_decode(ctx, head_dim, group, n_kv, ctx_len,
     dev.close()
 
 
+@pytest.mark.parametrize("head_dim,group,n_kv,ctx_len,n_new", [
+    (64, 4, 4, 1000, 513),    # two query heads per wave of V
+    (128, 4, 4, 1500, 257),
+    (64, 4, 4, 900, 1025),    # four
+    (128, 8, 2, 700, 513),    # four of eight
+])
+def test_batch_attention_heads_with_their_own_tiles(ctx, head_dim, group, n_kv, ctx_len, n_new):
+    """Softmaxes of a few positions each (queries of size ~400 against keys of
+    unit size), so the heads that share a wave of V seldom share a live tile:
+    the wave then takes them one after the other.  Against the same tokens
+    decoded one at a time: hidden state and cache bytes."""
+    cfg = bs.BitNetConfig(n_layers=2, n_embd=head_dim * group * n_kv, n_ff=384, n_heads=group * n_kv,
+                          n_kv_heads=n_kv, head_dim=head_dim, vocab=300, context_length=4096)
+    hm = bs.make_host_model(cfg, seed=head_dim + n_new)
+    for hl in hm.layers:
+        hl.scales["attn_q"] *= 10.0
+        hl.scales["attn_k"] = 1.0 / np.sqrt(cfg.n_embd * 2 / 3)
+    dev = bs.load_device_model(ctx, hm)
+    toks = np.random.default_rng(n_new).integers(0, cfg.vocab, n_new).tolist()
+    a, b = dev.kv_cache(ctx_len + n_new), dev.kv_cache(ctx_len + n_new)
+    k, v = bs.kv_prefill(cfg, seed=9, n_pos=ctx_len)
+    a.append_positions(k, v)
+    b.append_positions(k, v)
+    hidden, _ = dev.batch_forward([a], [toks])
+    for t in toks:
+        hb = b.forward(t, b.position)
+    assert bits_equal(hidden[0], hb)
+    for l in range(cfg.n_layers):
+        assert all(np.array_equal(x, y) for x, y in zip(a.read_raw(l, a.position), b.read_raw(l, b.position)))
+    a.close()
+    b.close()
+    dev.close()
+
+
 def test_batch_over_64_tokens(pair):
     # more than one 64-token GEMM tile, tiles shared by several sequences
     cfg, hm, dev, orm = pair
