@@ -41,6 +41,7 @@
 
 #include "wm_internal.h"
 #include "wm_seqsum.h"
+#include "wm_terms.h"
 
 namespace {
 
@@ -117,35 +118,22 @@ __device__ __forceinline__ float key_value(uint32_t k) {
 constexpr uint32_t kKeyPosZero = 0x80000000u, kKeyNegZero = 0x7fffffffu;
 
 // Sources of left-to-right sums: f(i) is term i, f.get8(i, n, v) terms
-// i .. i+7 (i a multiple of 8; zeros from n on) from 32-byte aligned arrays.
+// i .. i+7 (wm::terms_get8).
 struct plain_terms {
     const float *a;
     __device__ __forceinline__ float map(float x, uint32_t) const { return x; }
     __device__ __forceinline__ float operator()(uint32_t i) const { return a[i]; }
-    __device__ __forceinline__ void get8(uint32_t i, uint32_t n, float (&v)[8]) const;
-};
-template <typename F>
-__device__ __forceinline__ void terms_get8(const F &f, const float *a, uint32_t i, uint32_t n, float (&v)[8]) {
-    if (i + 8 <= n) {
-        const float4 x = *reinterpret_cast<const float4 *>(a + i), y = *reinterpret_cast<const float4 *>(a + i + 4);
-        const float r[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = f.map(r[j], i + j);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = i + j < n ? f.map(a[i + j], i + j) : 0.0f;
+    __device__ __forceinline__ void get8(uint32_t i, uint32_t n, float (&v)[8]) const {
+        wm::terms_get8(*this, a, i, n, v);
     }
-}
-__device__ __forceinline__ void plain_terms::get8(uint32_t i, uint32_t n, float (&v)[8]) const {
-    terms_get8(*this, a, i, n, v);
-}
+};
 // values held as order keys (the sorted probabilities)
 struct key_terms {
     const uint32_t *k;
     __device__ __forceinline__ float map(float x, uint32_t) const { return key_value(__float_as_uint(x)); }
     __device__ __forceinline__ float operator()(uint32_t i) const { return key_value(k[i]); }
     __device__ __forceinline__ void get8(uint32_t i, uint32_t n, float (&v)[8]) const {
-        terms_get8(*this, reinterpret_cast<const float *>(k), i, n, v);
+        wm::terms_get8(*this, reinterpret_cast<const float *>(k), i, n, v);
     }
 };
 // probabilities exp * inv after top-p (entries at or after the cut's last
@@ -162,7 +150,9 @@ struct prob_terms {
         return keep ? p * inv2 : 0.0f;
     }
     __device__ __forceinline__ float operator()(uint32_t i) const { return map(e[i], i); }
-    __device__ __forceinline__ void get8(uint32_t i, uint32_t n, float (&v)[8]) const { terms_get8(*this, e, i, n, v); }
+    __device__ __forceinline__ void get8(uint32_t i, uint32_t n, float (&v)[8]) const {
+        wm::terms_get8(*this, e, i, n, v);
+    }
 };
 
 // argmax as lm_head.rs:161-174 (`if v > best`, starting from a[0]): index 0
@@ -173,11 +163,11 @@ __device__ uint32_t block_argmax_first(const F &a, uint32_t n, float *rv, uint32
     const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     float bv = -INFINITY;
     uint32_t bi = 0xffffffffu;
-    for (uint32_t i = tid; i < n; i += kSampleThreads) {
-        const float v = a(i);
+    for (uint64_t i = tid; i < n; i += kSampleThreads) {  // (i passes 2^32 where n is close to it)
+        const float v = a((uint32_t)i);
         if (!isnan(v) && (bi == 0xffffffffu || v > bv)) {
             bv = v;
-            bi = i;
+            bi = (uint32_t)i;
         }
     }
     for (int o = 32; o > 0; o >>= 1) {
