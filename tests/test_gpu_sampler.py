@@ -160,6 +160,12 @@ def test_rollback_restores_history_and_rng(ctx):  # sampler.rs:348-372 on the de
     ("normal", 2048, dict(top_k=30, top_p=0.0)),
     ("normal", 2048, dict(top_k=30, top_p=NAN)),
     ("normal", 70001, dict(top_k=3000, top_p=0.9)),
+    # the longest list, and one value more: all values sorted
+    ("normal", 9000, dict(top_k=3840)),
+    ("normal", 9000, dict(top_k=3841)),
+    ("normal", 70001, dict(top_k=3841, top_p=0.9)),
+    ("normal", 9000, dict(top_k=8999, top_p=0.0)),
+    ("normal", 9000, dict(top_k=5000, top_p=NAN)),
     ("wide", 5000, dict(top_k=64, top_p=0.95)),       # exps that underflow among the kept
     # ties at the threshold: within the list, and more than it holds
     ("ties", 3000, dict(top_k=40, top_p=0.5)),
@@ -207,6 +213,27 @@ def test_sample_routes_match_oracle(ctx, kind, n, kw):
         assert dev.checkpoint()[0] == ref.state.value
         dev.observe(got)
         ref.observe(want)
+
+
+@pytest.mark.parametrize("top_k", [40, 3840, 3841])
+@pytest.mark.parametrize("top_p", [None, 0.9, 0.0, NAN])
+def test_nan_under_top_k_on_either_route(ctx, top_k, top_p):
+    """A NaN among the values top-k orders is refused by the list and by the
+    sort alike, the state unchanged, and the next draw is as if it had not
+    been."""
+    n = 9000
+    dev, ref = pair_samplers(ctx, 17, temperature=1.0, top_k=top_k, top_p=top_p)
+    rng = np.random.default_rng(top_k)
+    for _ in range(2):
+        logits = rng.standard_normal(n).astype(np.float32)
+        bad = logits.copy()
+        bad[n // 2] = np.nan
+        before = dev.checkpoint()[0]
+        with pytest.raises(wh.WillametteError) as ei:
+            dev.sample(bad)
+        assert ei.value.kind == "NonFinite" and dev.checkpoint()[0] == before
+        assert dev.sample(logits) == ref.sample(logits)
+        assert dev.checkpoint()[0] == ref.state.value
 
 
 # ---- batched prefill and the sampled loop --------------------------------
