@@ -469,7 +469,7 @@ __global__ __launch_bounds__(kFinalThreads) void k_argmax_final(const argcand *_
                                const float *__restrict__ first_logit, uint32_t *__restrict__ out) {
     float bv = -INFINITY;
     uint32_t bi = 0xFFFFFFFFu;
-    for (uint32_t i = threadIdx.x; i < n_cands; i += kFinalThreads)
+    for (uint32_t i = threadIdx.x; i < n_cands; i += blockDim.x)
         if (cand_better(cands[i].v, cands[i].i, bv, bi)) {
             bv = cands[i].v;
             bi = cands[i].i;
@@ -486,7 +486,7 @@ __global__ __launch_bounds__(kFinalThreads) void k_argmax_final(const argcand *_
     if ((threadIdx.x & 63) == 0) s_c[threadIdx.x >> 6] = argcand{bv, bi};
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int i = 1; i < kFinalThreads / 64; i++)
+        for (uint32_t i = 1; i < blockDim.x / 64; i++)
             if (cand_better(s_c[i].v, s_c[i].i, bv, bi)) {
                 bv = s_c[i].v;
                 bi = s_c[i].i;
@@ -1341,9 +1341,12 @@ void wm_launch_q6k_logits_argmax(const uint8_t *w, uint32_t n_blocks, uint32_t n
         WM_LOGITS_CASE(2) default: WM_LOGITS_CASE(1)
     }
 #undef WM_LOGITS_CASE
+    // One wave for up to 64 maxima (300 to 1000 rows: 16.7 us a call, with
+    // eight waves 17.0); for the 768 of a large table eight take 4 us where
+    // one took 10 for 1536.
     if (argmax_out)
-        hipLaunchKernelGGL(k_argmax_final, dim3(1), dim3(kFinalThreads), 0, s, cands, blocks, logits,
-                           argmax_out);
+        hipLaunchKernelGGL(k_argmax_final, dim3(1), dim3(blocks <= 64 ? 64 : kFinalThreads), 0, s, cands, blocks,
+                           logits, argmax_out);
 }
 
 // Argmax only: the bounded pass, then selection + exact rescoring + argmax

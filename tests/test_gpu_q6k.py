@@ -110,6 +110,23 @@ def test_argmax_rules_on_device(ctx):
     assert a == 2
 
 
+@pytest.mark.parametrize("n_rows", [1024, 1025, 8193, 12289])
+def test_argmax_over_the_workgroups_maxima(ctx, n_rows):
+    """The id where the maximum of the workgroups' maxima changes its number
+    of threads (1024 rows: 64 maxima) or of values per thread: the best row
+    last, then a tie with the first."""
+    raw = np.tile(ones_block(1), n_rows).reshape(n_rows, 210)
+    raw[-1] = ones_block(2)
+    h = np.ones(256, np.float32)
+    t = ctx.upload_q6k(raw.ravel(), 256, n_rows)
+    assert wh.logits_argmax(ctx, t, h)[1] == n_rows - 1
+    t.close()
+    raw[0] = ones_block(2)
+    t = ctx.upload_q6k(raw.ravel(), 256, n_rows)
+    assert wh.logits_argmax(ctx, t, h)[1] == 0
+    t.close()
+
+
 def test_nonfinite_scale_blocks_match_oracle(ctx):
     rng = np.random.default_rng(9)
     raw = random_q6k(rng, 64, 512, finite=True).reshape(-1, 210)
