@@ -517,6 +517,16 @@ wm_status wm_debug_rerun_role(wm_model *m, wm_kv_cache *kv, uint32_t layer, uint
 #define WM_FUSED_DEBUG_ATTN_LOOSE_COUNT 16u
 wm_status wm_debug_set_fused_flags(wm_ctx *ctx, uint32_t flags);
 
+/* No counterpart in the reference: the kernels wm_batch_forward would choose
+ * for the attention of n_seqs sequences of contexts[i] positions with n_new[i]
+ * tokens each (host-only), so that tests can say which ones they run:
+ * plan[0] tokens per work item of the scores (the most any item has),
+ * plan[1] waves per row of the softmax, plan[2] float4s of a row per lane,
+ * plan[3] query heads per wave of V. */
+wm_status wm_debug_batch_plan(const uint32_t *contexts, const uint32_t *n_new, uint32_t n_seqs,
+                              uint32_t n_kv_heads, uint32_t group, uint32_t head_dim,
+                              uint32_t *plan);
+
 /* ---- synthetic BitNet-shaped inputs (src/synth.rs) ------------------- */
 
 /* Counter-based SplitMix64 streams, identical on every host: value i of

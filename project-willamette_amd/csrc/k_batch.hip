@@ -1479,6 +1479,14 @@ uint32_t wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t n_kv_he
     return heads;
 }
 
+// Waves per row: one where a batch has rows enough to fill the chip, four
+// for few rows of more than 1024 positions (each CU then holds eight).
+wm_attn_softmax_plan wm_attn_rows_softmax_plan(uint32_t n_rows, uint32_t n_max) {
+    wm_attn_softmax_plan p{n_max <= 1024 || n_rows > 8 * kGemmCus ? 1u : 4u, 1u};
+    while (256 * p.waves * p.slots < n_max) p.slots *= 2;
+    return p;
+}
+
 void wm_launch_attn_rows(const float *q, const wm_batch_tok *tok, uint32_t m, uint32_t n_max,
                          uint32_t layer, uint32_t n_kv_heads, uint32_t head_dim, uint32_t group,
                          float scale, float *scores, float *out, uint32_t n_sc, uint32_t n_sv,
@@ -1497,13 +1505,10 @@ void wm_launch_attn_rows(const float *q, const wm_batch_tok *tok, uint32_t m, ui
     WM_SCORES_CASE(64, 1) WM_SCORES_CASE(64, 2) WM_SCORES_CASE(64, 4) WM_SCORES_CASE(64, 8)
 #undef WM_SCORES_CASE
     const uint32_t n_rows = m * n_heads;
-    // Waves per row: one where a batch has rows enough to fill the chip, four
-    // for few rows of more than 1024 positions (each CU then holds eight).
-    const uint32_t wpr = n_max <= 1024 || n_rows > 8 * kGemmCus ? 1 : 4;
-    const uint32_t f4 = (n_max + 256 * wpr - 1) / (256 * wpr);
+    const wm_attn_softmax_plan sp = wm_attn_rows_softmax_plan(n_rows, n_max);
     const dim3 sm_grid((n_rows + kSmRows - 1) / kSmRows);
 #define WM_SM_CASE(W, F)                                                                       \
-    if (wpr == W && f4 <= F && f4 > F / 2)                                                     \
+    if (sp.waves == W && sp.slots == F)                                                        \
         hipLaunchKernelGGL((k_attn_softmax_rows<W, F>), sm_grid, dim3(kSmRows * W * 64), 0, s, a, n_rows);
     WM_SM_CASE(1, 1) WM_SM_CASE(1, 2) WM_SM_CASE(1, 4) WM_SM_CASE(1, 8) WM_SM_CASE(1, 16)
     WM_SM_CASE(4, 2) WM_SM_CASE(4, 4)

@@ -592,6 +592,30 @@ wm_status wm_batch_forward(wm_model *m, wm_kv_cache *const *caches, uint32_t n_s
     return WM_OK;
 }
 
+wm_status wm_debug_batch_plan(const uint32_t *contexts, const uint32_t *n_new, uint32_t n_seqs,
+                              uint32_t n_kv_heads, uint32_t group, uint32_t head_dim, uint32_t *plan) {
+    if (!contexts || !n_new || !plan || !n_seqs || !n_kv_heads || !wm_attn_rows_supported(head_dim, group)) return WM_E_ARG;
+    std::vector<wm_batch_tok> tok;
+    uint32_t n_max = 0;
+    for (uint32_t i = 0; i < n_seqs; i++) {
+        if (!n_new[i] || tok.size() + n_new[i] > kBatchMaxTokens || contexts[i] + (uint64_t)n_new[i] > 4096) return WM_E_SHAPE;
+        // (the plan tells caches apart by their address and reads none)
+        int8_t *const cache = reinterpret_cast<int8_t *>((uintptr_t)(i + 1));
+        for (uint32_t j = 0; j < n_new[i]; j++)
+            tok.push_back(wm_batch_tok{cache, nullptr, nullptr, nullptr, 4096, contexts[i] + j});
+        n_max = std::max(n_max, contexts[i] + n_new[i]);
+    }
+    const uint32_t m = (uint32_t)tok.size();
+    std::vector<wm_attn_item> sc, sv;
+    plan[3] = wm_attn_rows_plan(tok.data(), m, n_kv_heads, group, head_dim, sc, sv);
+    plan[0] = 0;
+    for (const wm_attn_item &it : sc) plan[0] = std::max(plan[0], it.nt);
+    const wm_attn_softmax_plan p = wm_attn_rows_softmax_plan(m * n_kv_heads * group, n_max);
+    plan[1] = p.waves;
+    plan[2] = p.slots;
+    return WM_OK;
+}
+
 wm_status wm_model_create(wm_ctx *ctx, const wm_model_config *cfg, wm_model **out) {
     if (!ctx || !cfg || !out) return WM_E_ARG;
     *out = nullptr;

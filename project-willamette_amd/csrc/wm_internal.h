@@ -577,6 +577,11 @@ struct wm_attn_item {
 // where they can.  Returns the query heads per V row set.
 uint32_t wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t n_kv_heads, uint32_t group,
                            uint32_t head_dim, std::vector<wm_attn_item> &sc, std::vector<wm_attn_item> &sv);
+// Waves per row of the softmax, and float4s of it per lane (a power of two).
+struct wm_attn_softmax_plan {
+    uint32_t waves, slots;
+};
+wm_attn_softmax_plan wm_attn_rows_softmax_plan(uint32_t n_rows, uint32_t n_max);
 // The V kernel reads a tile of this many positions past a cache's last one.
 constexpr uint32_t WM_ATTN_TILE = 64;
 // Device workspace of one step: scores, live-tile flags and the n_items work

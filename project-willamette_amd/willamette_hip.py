@@ -137,6 +137,7 @@ EXPORTS = {
     "wm_bitlinear_i2s_matvec_f32_dev_noalloc": (C.c_int, _vp, _vp, _vp, _vp),
     "wm_debug_rerun_role": (C.c_int, _vp, _vp, C.c_uint32, C.c_uint32, C.c_uint32),
     "wm_debug_set_fused_flags": (C.c_int, _vp, C.c_uint32),
+    "wm_debug_batch_plan": (C.c_int, _u32p, _u32p, C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, _u32p),
     "wm_bitlinear_i2s_matvec_f32_multi_dev": (C.c_int, _vp, C.POINTER(_vp), C.c_uint32, _vp, _vp),
     "wm_bitlinear_i2s_matmul_f32_dev": (C.c_int, _vp, _vp, _vp, C.c_uint32, _vp),
     "wm_bitlinear_i2s_matmul_f32": (C.c_int, _vp, _vp, _f32p, C.c_size_t, C.c_uint32, _f32p,
@@ -497,6 +498,16 @@ def debug_seq_sum(ctx: Context, values: np.ndarray) -> np.float32:
     out = C.c_float()
     ctx.check(lib.wm_debug_seq_sum(ctx.h, _ptr(values, C.c_float), values.size, C.byref(out)))
     return np.float32(out.value)
+
+
+def debug_batch_plan(contexts, n_new, n_kv_heads: int, group: int, head_dim: int) -> dict:
+    c, n = np.asarray(contexts, np.uint32), np.asarray(n_new, np.uint32)
+    plan = np.zeros(4, np.uint32)
+    st = lib.wm_debug_batch_plan(_ptr(c, C.c_uint32), _ptr(n, C.c_uint32), c.size, n_kv_heads, group, head_dim,
+                                 _ptr(plan, C.c_uint32))
+    if st:
+        raise WillametteError(st, "debug_batch_plan")
+    return dict(zip(("scores_tokens", "softmax_waves", "softmax_slots", "v_heads"), plan.tolist()))
 
 
 def q6k_dequantize_row(ctx: Context, t: Tensor, row: int) -> np.ndarray:

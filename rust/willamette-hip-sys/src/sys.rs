@@ -175,6 +175,7 @@ extern "C" {
     pub fn wm_debug_q6k_bounded_logits_dev(ctx: *mut wm_ctx, token_embd: *const wm_tensor, d_hidden: *const f32, d_approx: *mut f32, d_bound: *mut f32, reuse_prep: c_int) -> wm_status;
     pub fn wm_debug_rerun_role(m: *mut wm_model, kv: *mut wm_kv_cache, layer: u32, role: u32, reps: u32) -> wm_status;
     pub fn wm_debug_set_fused_flags(ctx: *mut wm_ctx, flags: u32) -> wm_status;
+    pub fn wm_debug_batch_plan(contexts: *const u32, n_new: *const u32, n_seqs: u32, n_kv_heads: u32, group: u32, head_dim: u32, plan: *mut u32) -> wm_status;
     pub fn wm_synth_stream_seed(seed: u64, tag: u64) -> u64;
     pub fn wm_synth_i2s(seed: u64, tag: u64, packed: *mut u8, n_bytes: usize);
     pub fn wm_synth_normal(seed: u64, tag: u64, out: *mut f32, n: usize, sigma: f64);

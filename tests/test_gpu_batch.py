@@ -193,24 +193,46 @@ def test_batch_dense_softmax_long_rows(ctx):
     orm.close()
 
 
-@pytest.mark.parametrize("head_dim,group,n_kv,ctx_len,n_new,dense", [
-    # (rows' ends at 256, 512, 1024 and 2048 positions: the softmax's sizes;
-    # group and tokens: query heads and rows per wave of scores and V)
-    (64, 1, 4, 0, 3, True),
-    (64, 8, 1, 250, 9, True),
-    (64, 2, 2, 505, 11, True),
-    (128, 2, 1, 1020, 7, True),
-    (128, 8, 1, 2043, 8, False),
-    (128, 1, 4, 4070, 26, True),       # the last tile reaches past the context
-    (128, 4, 2, 63, 129, True),
-    (128, 4, 4, 0, 512, True),         # four heads per wave of V
-    (64, 4, 4, 1000, 300, False),      # two
-])
-def test_batch_attention_sizes_match_decode(ctx, head_dim, group, n_kv, ctx_len, n_new, dense):
+# (head_dim, query heads per KV head, KV heads, context, new tokens, dense
+# softmaxes, plan): rows' ends at 256, 512, 1024 and 2048 positions (the
+# softmax's sizes), and what the plan chooses for the batch: tokens per work
+# item of the scores, waves per row and float4s per lane of the softmax, query
+# heads per wave of V
+ATTENTION_CASES = [
+    (64, 1, 4, 0, 3, True, (1, 1, 1, 1)),
+    (64, 8, 1, 250, 9, True, (1, 1, 2, 1)),
+    (64, 2, 2, 505, 11, True, (1, 1, 4, 1)),
+    (128, 2, 1, 1020, 7, True, (1, 4, 2, 1)),
+    (128, 8, 1, 2043, 8, False, (1, 4, 4, 1)),
+    (128, 1, 4, 4064, 26, True, (2, 4, 4, 1)),    # the last tile reaches past the cache's 4090 positions
+    (128, 4, 2, 63, 129, True, (1, 1, 1, 1)),
+    (128, 4, 4, 0, 512, True, (2, 1, 2, 4)),
+    (64, 4, 4, 1000, 300, False, (4, 1, 8, 1)),
+    # heads that share a wave of V, the last workgroup's share ragged
+    (64, 4, 4, 1000, 513, False, (8, 1, 8, 2)),
+    (64, 4, 4, 900, 1025, True, (8, 1, 8, 4)),
+    (128, 4, 4, 1500, 257, True, (8, 1, 8, 2)),
+    (128, 8, 2, 700, 513, True, (4, 1, 8, 4)),
+    # more than 2048 long dense rows: one wave each, two to four rounds of its sum
+    (64, 4, 4, 1501, 151, True, (4, 1, 8, 1)),
+    (64, 4, 4, 3001, 151, True, (8, 1, 16, 1)),
+    # eight tokens per item of the scores, five in the last (with one query
+    # head per KV head, not a multiple of the four rows of a step)
+    (64, 1, 16, 3700, 29, True, (8, 4, 4, 1)),
+    (64, 2, 16, 3700, 29, True, (8, 4, 4, 1)),
+    (64, 8, 4, 3700, 109, True, (8, 1, 16, 1)),
+    (128, 1, 16, 3500, 29, True, (8, 4, 4, 1)),
+    (128, 2, 8, 3500, 61, True, (8, 4, 4, 1)),
+]
+
+
+@pytest.mark.parametrize("head_dim,group,n_kv,ctx_len,n_new,dense,plan", ATTENTION_CASES)
+def test_batch_attention_sizes_match_decode(ctx, head_dim, group, n_kv, ctx_len, n_new, dense, plan):
     """One sequence's tokens in a batch against the same tokens decoded one at
     a time (checked against the oracle elsewhere): hidden state and cache
     bytes, the second layer's of every token among them."""
     n_embd = head_dim * group * n_kv
+    assert tuple(wh.debug_batch_plan([ctx_len], [n_new], n_kv, group, head_dim).values()) == plan
     cfg = bs.BitNetConfig(n_layers=2, n_embd=n_embd, n_ff=384, n_heads=group * n_kv, n_kv_heads=n_kv,
                           head_dim=head_dim, vocab=300, context_length=4096)
     hm = bs.make_host_model(cfg, seed=head_dim + group)
@@ -220,7 +242,7 @@ def test_batch_attention_sizes_match_decode(ctx, head_dim, group, n_kv, ctx_len,
     dev = bs.load_device_model(ctx, hm)
     rng = np.random.default_rng(ctx_len + n_new)
     toks = rng.integers(0, cfg.vocab, n_new).tolist()
-    a, b = dev.kv_cache(4096), dev.kv_cache(4096)
+    a, b = dev.kv_cache(ctx_len + n_new), dev.kv_cache(ctx_len + n_new)
     if ctx_len:
         k, v = bs.kv_prefill(cfg, seed=9, n_pos=ctx_len)
         a.append_positions(k, v)
@@ -236,17 +258,18 @@ def test_batch_attention_sizes_match_decode(ctx, head_dim, group, n_kv, ctx_len,
     dev.close()
 
 
-@pytest.mark.parametrize("head_dim,group,n_kv,ctx_len,n_new", [
-    (64, 4, 4, 1000, 513),    # two query heads per wave of V
-    (128, 4, 4, 1500, 257),
-    (64, 4, 4, 900, 1025),    # four
-    (128, 8, 2, 700, 513),    # four of eight
+@pytest.mark.parametrize("head_dim,group,n_kv,ctx_len,n_new,v_heads", [
+    (64, 4, 4, 1000, 513, 2),
+    (128, 4, 4, 1500, 257, 2),
+    (64, 4, 4, 900, 1025, 4),
+    (128, 8, 2, 700, 513, 4),
 ])
-def test_batch_attention_heads_with_their_own_tiles(ctx, head_dim, group, n_kv, ctx_len, n_new):
+def test_batch_attention_heads_with_their_own_tiles(ctx, head_dim, group, n_kv, ctx_len, n_new, v_heads):
     """Softmaxes of a few positions each (queries of size ~400 against keys of
     unit size), so the heads that share a wave of V seldom share a live tile:
     the wave then takes them one after the other.  Against the same tokens
     decoded one at a time: hidden state and cache bytes."""
+    assert wh.debug_batch_plan([ctx_len], [n_new], n_kv, group, head_dim)["v_heads"] == v_heads
     cfg = bs.BitNetConfig(n_layers=2, n_embd=head_dim * group * n_kv, n_ff=384, n_heads=group * n_kv,
                           n_kv_heads=n_kv, head_dim=head_dim, vocab=300, context_length=4096)
     hm = bs.make_host_model(cfg, seed=head_dim + n_new)
