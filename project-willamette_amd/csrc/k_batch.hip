@@ -1480,7 +1480,14 @@ uint32_t wm_attn_rows_plan(const wm_batch_tok *tok, uint32_t m, uint32_t n_kv_he
 }
 
 // Waves per row: one where a batch has rows enough to fill the chip, four
-// for few rows of more than 1024 positions (each CU then holds eight).
+// for few rows of more than 1024 positions.  The line is where the four-wave
+// workgroups (1024 threads, four rows) no longer all fit at once, two to a CU:
+// us with one wave and with four, at 640 / 1920 / 2080 / 5120 rows of 1100
+// positions 11 and 10 / 13.0 and 12.8 / 14 and 18.5 / 25 and 28; of 3000
+// 24 and 18 / 28 and 23 / 29 and 35 / 55 and 54; of 3850 30 and 22 / 35 and 28 /
+// 36 and 44 / 68 and 68.  Both numbers are the batch's, its longest row's and
+// the rows of all: one row of 3900 positions among short ones is taken as
+// if all were long, 2560 such rows 29 where four waves would take 21.
 wm_attn_softmax_plan wm_attn_rows_softmax_plan(uint32_t n_rows, uint32_t n_max) {
     wm_attn_softmax_plan p{n_max <= 1024 || n_rows > 8 * kGemmCus ? 1u : 4u, 1u};
     while (256 * p.waves * p.slots < n_max) p.slots *= 2;
