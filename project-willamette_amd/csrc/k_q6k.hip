@@ -465,11 +465,12 @@ __global__ __launch_bounds__(kLogitsBlock, 3) void k_q6k_logits(
 
 // Combine the per-block candidates; a NaN logit at index 0 wins, as the
 // reference's scan starts from logits[0] and NaN compares false.
-__global__ __launch_bounds__(kFinalThreads) void k_argmax_final(const argcand *__restrict__ cands, uint32_t n_cands,
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_argmax_final(const argcand *__restrict__ cands, uint32_t n_cands,
                                const float *__restrict__ first_logit, uint32_t *__restrict__ out) {
     float bv = -INFINITY;
     uint32_t bi = 0xFFFFFFFFu;
-    for (uint32_t i = threadIdx.x; i < n_cands; i += blockDim.x)
+    for (uint32_t i = threadIdx.x; i < n_cands; i += THREADS)
         if (cand_better(cands[i].v, cands[i].i, bv, bi)) {
             bv = cands[i].v;
             bi = cands[i].i;
@@ -482,11 +483,11 @@ __global__ __launch_bounds__(kFinalThreads) void k_argmax_final(const argcand *_
             bi = oi;
         }
     }
-    __shared__ argcand s_c[kFinalThreads / 64];
+    __shared__ argcand s_c[THREADS / 64];
     if ((threadIdx.x & 63) == 0) s_c[threadIdx.x >> 6] = argcand{bv, bi};
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (uint32_t i = 1; i < blockDim.x / 64; i++)
+        for (int i = 1; i < THREADS / 64; i++)
             if (cand_better(s_c[i].v, s_c[i].i, bv, bi)) {
                 bv = s_c[i].v;
                 bi = s_c[i].i;
@@ -1343,10 +1344,15 @@ void wm_launch_q6k_logits_argmax(const uint8_t *w, uint32_t n_blocks, uint32_t n
 #undef WM_LOGITS_CASE
     // One wave for up to 64 maxima (300 to 1000 rows: 16.7 us a call, with
     // eight waves 17.0); for the 768 of a large table eight take 4 us where
-    // one took 10 for 1536.
-    if (argmax_out)
-        hipLaunchKernelGGL(k_argmax_final, dim3(1), dim3(blocks <= 64 ? 64 : kFinalThreads), 0, s, cands, blocks,
-                           logits, argmax_out);
+    // one took 10 for 1536.  (The number of threads is a constant of each: as a
+    // value the loop over the waves stays one, 0.25 us at 250 maxima.)
+    if (argmax_out) {
+        if (blocks <= 64)
+            hipLaunchKernelGGL(k_argmax_final<64>, dim3(1), dim3(64), 0, s, cands, blocks, logits, argmax_out);
+        else
+            hipLaunchKernelGGL(k_argmax_final<kFinalThreads>, dim3(1), dim3(kFinalThreads), 0, s, cands, blocks,
+                               logits, argmax_out);
+    }
 }
 
 // Argmax only: the bounded pass, then selection + exact rescoring + argmax
