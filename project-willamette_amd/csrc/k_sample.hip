@@ -426,8 +426,8 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample_greedy(sample_args a)
 // Repetition penalty (each history id once: a bit per value of the strip),
 // temperature, each workgroup's maximum and, for top-k, the histogram.
 // Bound by launch latency and one pass over the logits: 128256 values with
-// 600 history ids take 4.5-6 us (one workgroup took 100-120 us, the distinct
-// test over the history its largest part).
+// 600 history ids take 7.5-8.5 us in a kernel trace (one workgroup took
+// 100-120 us, the distinct test over the history its largest part).
 __global__ __launch_bounds__(kScanThreads) void k_sample_scan(sample_args a) {
     __shared__ uint32_t h[kBins];
     __shared__ uint32_t bits[kStrip / 32];
