@@ -173,6 +173,8 @@ def test_rollback_restores_history_and_rng(ctx):  # sampler.rs:348-372 on the de
     ("zeros", 3000, dict(top_k=10)),                  # +0 and -0 around the threshold
     ("zeros", 9000, dict(top_k=10, top_p=0.4)),
     ("neg_inf", 3000, dict(top_k=100, top_p=0.9)),    # fewer finite values than k
+    ("neg_inf", 9000, dict(top_k=100, top_p=0.9)),    # the same, more masked values than the list holds
+    ("neg_inf", 9000, dict(top_k=100)),
     # all values: chunks of 512 terms, rounds of 262144
     ("normal", 511, dict(top_p=0.9)),
     ("normal", 513, dict()),
