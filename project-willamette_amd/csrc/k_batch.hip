@@ -895,7 +895,7 @@ __global__ __launch_bounds__(kSmRows * WPR * 64) void k_attn_softmax_rows(attn_r
         const uint32_t k = i * WPR + part;
         if (256 * k < n) x[i] = reinterpret_cast<const float4 *>(w)[min(64 * k + lane, n4 - 1)];
     }
-    uint32_t n_max = 0;  // the workgroup's longest row (rows of one token or of two)
+    uint32_t n_max = 0;  // the workgroup's longest row (its rows are of one token or of a few)
 #pragma unroll
     for (uint32_t i = 0; i < kSmRows; i++)
         n_max = max(n_max, a.tok[min(row0 + i, n_rows - 1) / a.n_heads].pos + 1);

@@ -595,6 +595,7 @@ wm_status wm_batch_forward(wm_model *m, wm_kv_cache *const *caches, uint32_t n_s
 wm_status wm_debug_batch_plan(const uint32_t *contexts, const uint32_t *n_new, uint32_t n_seqs,
                               uint32_t n_kv_heads, uint32_t group, uint32_t head_dim, uint32_t *plan) {
     if (!contexts || !n_new || !plan || !n_seqs || !n_kv_heads || !wm_attn_rows_supported(head_dim, group)) return WM_E_ARG;
+    if ((uint64_t)n_kv_heads * group * head_dim > 8192) return WM_E_SHAPE;  // batch_forward's limit on n_embd
     std::vector<wm_batch_tok> tok;
     uint32_t n_max = 0;
     for (uint32_t i = 0; i < n_seqs; i++) {

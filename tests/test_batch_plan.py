@@ -37,7 +37,8 @@ def test_plan_of_several_sequences():
 
 @pytest.mark.parametrize("contexts,n_new,n_kv,group,head_dim", [
     ([], [], 5, 4, 128), ([1], [0], 5, 4, 128), ([4090], [7], 5, 4, 128), ([0], [16385], 5, 4, 128),
-    ([0xFFFFFFFF], [1], 5, 4, 128), ([1], [1], 0, 4, 128), ([1], [1], 5, 3, 128), ([1], [1], 5, 4, 96)])
+    ([0xFFFFFFFF], [1], 5, 4, 128), ([1], [1], 0, 4, 128), ([1], [1], 5, 3, 128), ([1], [1], 5, 4, 96),
+    ([1], [1], 0x80000000, 4, 128), ([1], [1], 17, 4, 128)])
 def test_plan_rejects(contexts, n_new, n_kv, group, head_dim):
     with pytest.raises(wh.WillametteError):
         wh.debug_batch_plan(contexts, n_new, n_kv, group, head_dim)
